@@ -1,4 +1,5 @@
-// Product-quantized KV decode attention, LUT build, PQ encode and k-means update.
+// Product-quantized KV decode attention, LUT build and k-means update (the PQ
+// encode is in pq_encode.hip).
 //
 // Replaces src/attention_kernels.py:
 //   decode_attn_pq_lut_kv  :397-500  LUT-scored keys, codebook-reconstructed values
@@ -1295,56 +1296,6 @@ __global__ __launch_bounds__(64) void pq_lut_kernel(const uint16_t* q, int64_t q
   }
 }
 
-// ============================================================================
-// Encode: idx[n, j] = argmin_c sum_e (x[n, 8j+e] - cb[j][c][e])^2, the sum in
-// fp32 in e order with separate multiply and add, first index on ties.
-// One thread per (vector, subspace); the head's codebook is staged in LDS.
-// ============================================================================
-constexpr int kEncThreads = 256;
-
-__global__ __launch_bounds__(kEncThreads) void pq_encode_kernel(const void* x, int x_dtype, int64_t rows_per_head,
-                                                                int64_t x_rs, const void* cb, int cb_f32,
-                                                                int64_t cb_sh, int M, int K, uint8_t* idx) {
-  __shared__ float cbs[16 * kPqKMax * 8];   // 128 KB: M <= 16 subspaces, K <= 256
-  const int head = blockIdx.y;
-  for (int e = threadIdx.x; e < M * K * 8; e += kEncThreads) {
-    const int64_t o = (int64_t)head * cb_sh + e;
-    cbs[e] = cb_f32 ? static_cast<const float*>(cb)[o] : (float)static_cast<const _Float16*>(cb)[o];
-  }
-  __syncthreads();
-  const int64_t gid = (int64_t)blockIdx.x * kEncThreads + threadIdx.x;
-  if (gid >= rows_per_head * M) return;
-  const int64_t n = gid / M;
-  const int j = (int)(gid - n * M);
-  const int64_t row = (int64_t)head * rows_per_head + n;
-  float xv[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const int64_t o = row * x_rs + j * 8 + e;
-    xv[e] = x_dtype == 0 ? bf16_bits_to_f32(static_cast<const uint16_t*>(x)[o])
-                         : (x_dtype == 1 ? (float)static_cast<const _Float16*>(x)[o] : static_cast<const float*>(x)[o]);
-  }
-  float best = __builtin_inff();
-  int bi = 0;
-  const float* cj = cbs + j * K * 8;
-  for (int c = 0; c < K; ++c) {
-    float dist = 0.f;
-    {
-#pragma clang fp contract(off)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float d = xv[e] - cj[c * 8 + e];
-        dist = dist + d * d;
-      }
-    }
-    if (dist < best) {
-      best = dist;
-      bi = c;
-    }
-  }
-  idx[row * M + j] = (uint8_t)bi;
-}
-
 // out[row, 8j + e] = cb[j][idx[row, j]][e] (ProductQuantizer.dequantize, src/quantization.py:213-226).
 __global__ void pq_decode_vectors_kernel(const uint8_t* idx, int64_t rows_per_head, const void* cb, int cb_f32,
                                          int64_t cb_sh, int M, int K, float* out) {
@@ -1647,21 +1598,6 @@ int bytes_pq_build_lut(const void* q, const void* cb, void* lut, int B, int Hq, 
   hipLaunchKernelGGL(pq_lut_kernel, dim3((unsigned)waves), dim3(64), 0, static_cast<hipStream_t>(stream),
                      static_cast<const uint16_t*>(q), q_sb, q_sh, static_cast<const _Float16*>(cb), cb_sh, Hk, G, HB,
                      M, K, scale, static_cast<float*>(lut));
-  return (int)hipGetLastError();
-}
-
-int bytes_pq_encode(const void* x, int x_dtype, int heads, int64_t rows_per_head, int64_t x_row_stride, int D,
-                    const void* cb, int cb_f32, int64_t cb_sh, int K, void* idx, void* stream) {
-  if (!x || !cb || !idx || heads <= 0 || rows_per_head < 0 || D % 8 != 0 || D / 8 > 16 || K <= 0 || K > kPqKMax)
-    return (int)hipErrorInvalidValue;
-  if (x_dtype < 0 || x_dtype > 2 || heads > 65535) return (int)hipErrorInvalidValue;
-  if (rows_per_head == 0) return 0;
-  const int M = D / 8;
-  const int64_t blocks = (rows_per_head * M + kEncThreads - 1) / kEncThreads;
-  if (blocks > 0x7FFFFFFFL) return (int)hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL(pq_encode_kernel, dim3((unsigned)blocks, (unsigned)heads), dim3(kEncThreads), 0,
-                     static_cast<hipStream_t>(stream), x, x_dtype, rows_per_head, x_row_stride, cb, cb_f32 ? 1 : 0,
-                     cb_sh, M, K, static_cast<uint8_t*>(idx));
   return (int)hipGetLastError();
 }
 

@@ -58,6 +58,55 @@ def test_encode_bit_exact(dev, dtype):
     assert torch.equal(goth, refh)
 
 
+@pytest.mark.parametrize("K,M,xdt,cdt", [
+    (256, 16, torch.bfloat16, torch.float16), (255, 16, torch.float16, torch.float16), (129, 3, torch.float32,
+    torch.float32), (65, 8, torch.float32, torch.float16), (64, 16, torch.bfloat16, torch.float32),
+    (33, 1, torch.float16, torch.float32), (3, 16, torch.bfloat16, torch.float16), (1, 5, torch.float32, torch.float32)])
+def test_encode_ranked_equals_full_search(dev, K, M, xdt, cdt):
+    """The ranked search equals the full evaluation for every input: ordinary
+    vectors, near and exact ties, codewords themselves, vectors far outside the
+    codebook, tiny and huge codebooks, infinities and NaN; rows that are no
+    multiple of a 32-row block, and rows that start off 16-byte boundaries."""
+    g = torch.Generator().manual_seed(K * 31 + M)
+    N = 677
+    cb = torch.randn(8, M, K, 8, generator=g)
+    cb[1, :, K // 2] = cb[1, :, 0]                        # duplicates: the first index wins
+    cb[2] = cb[2, :, :1] + 1e-3 * cb[2]                   # codewords closer than the ranking resolves
+    cb[3] *= 1e-6 if cdt == torch.float16 else 1e-25
+    cb[4] *= 1e4 if cdt == torch.float16 else 1e25
+    cb[5, :, K - 1] = float("inf")
+    cb[6, :, K // 3, 3] = float("nan")
+    cb[7] = cb[7].round()                                 # a lattice: many exact ties
+    cb = cb.to(cdt)
+    x = torch.randn(8, N, M * 8, generator=g)
+    x *= cb.float().nan_to_num(1, 1, 1).abs().amax(dim=(1, 2, 3)).clamp_min(1e-30)[:, None, None] / 3
+    x[:, 5] = cb[:, :, K - 1].float().reshape(8, -1)      # exact codewords
+    x[:, 6] = 0.5 * (cb[:, :, 0].float() + cb[:, :, K // 2].float()).reshape(8, -1)   # midway
+    x[:, 7] *= 100
+    x[:, 8] *= 1e6
+    x[:, 9, ::3] = float("inf")
+    x[:, 10, 1::5] = float("nan")
+    x[7, 20:] = x[7, 20:].round() + 0.5
+    x = x.to(xdt)
+
+    def full(xh, ch):                                     # strict "<" against +inf, in index order
+        xs, c = xh.float().reshape(-1, M, 1, 8), ch.float().unsqueeze(0)
+        d = torch.zeros(xs.shape[0], M, K)
+        for e in range(8):
+            t = xs[..., e] - c[..., e]
+            d = d + t * t
+        d = torch.where(d < float("inf"), d, torch.full_like(d, float("inf")))
+        return d.argmin(-1)
+
+    want = torch.stack([full(x[h], cb[h]) for h in range(8)])
+    assert torch.equal(PQ.pq_encode(x.to(dev), cb.to(dev)).cpu().long(), want)
+    wide = torch.zeros(8, N, M * 8 + 3, dtype=xdt)
+    wide[:, :, 1:M * 8 + 1] = x
+    for h in (0, 7):
+        assert torch.equal(PQ.pq_encode(wide.to(dev)[h, :, 1:M * 8 + 1], cb[h].to(dev)).cpu().long(), want[h])
+        assert torch.equal(PQ.pq_encode(x[h, :1].to(dev), cb[h].to(dev)).cpu().long(), want[h, :1])
+
+
 def test_decode_vectors_exact(dev):
     cb = _rand_cb((16, 256, 8), 6, torch.float32)
     g = torch.Generator().manual_seed(7)
