@@ -35,6 +35,46 @@ def test_pack_bit_exact(dev, bits, dtype):
 
 
 @pytest.mark.parametrize("bits", [2, 4])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shape", [(1, 32), (1, 2048), (3, 2080), (129, 96), (16, 4064)])
+def test_pack_flat_equals_general(dev, bits, dtype, shape):
+    """Gapless rows from a 16-byte boundary take the flat kernel, others the
+    one-thread-per-group kernel: the same bits for ordinary groups (which the
+    oracle pins too), quotients at and next to halves, constant groups, ranges
+    past fp16's and fp32's ends, infinities and NaN, in waves of 2048 elements
+    that are full, partial or alone."""
+    g = torch.Generator().manual_seed(shape[1] + bits)
+    x = torch.randn(*shape, generator=g) * 3
+    grp = x.reshape(-1, 32)
+    n = grp.shape[0]
+    L = 2 ** bits - 1
+    half = torch.arange(32) % L + 0.5                      # halves, then their neighbours
+    for i, f in enumerate((1.0, 1 + 2 ** -23, 1 - 2 ** -23, 1 + 2 ** -20)):
+        if n > i + 1:
+            t = half * f * 0.37
+            t[0], t[1] = 0.0, L * 0.37
+            grp[i + 1] = t
+    if n > 12:
+        grp[7] = 1.25
+        grp[8] *= 1e30
+        grp[9] *= 1e-30
+        grp[10] *= 3e38
+    want = R.kivi_quantize_and_pack_last_dim(x.to(dtype).nan_to_num(0, 1, -1), 32, bits)
+    got = K.quantize_and_pack_along_last_dim(x.to(dtype).nan_to_num(0, 1, -1).to(dev), 32, bits)
+    assert all(torch.equal(a.cpu(), b) for a, b in zip(got, want))   # (a minimum of both zeros may be either)
+    grp[0, 3], grp[0, 9] = float("inf"), float("nan")
+    if n > 12:
+        grp[11, ::2] = float("-inf")
+        grp[12] = float("nan")
+    x = x.to(dtype)
+    off = torch.zeros(x.numel() + 1, dtype=dtype, device=dev)
+    off[1:] = x.reshape(-1).to(dev)
+    slow = K.quantize_and_pack_along_last_dim(off[1:].reshape(shape), 32, bits)
+    fast = K.quantize_and_pack_along_last_dim(x.to(dev), 32, bits)
+    assert all(torch.equal(a.view(torch.int16), b.view(torch.int16)) for a, b in zip(fast, slow))
+
+
+@pytest.mark.parametrize("bits", [2, 4])
 def test_unpack_and_dequant(dev, bits):
     g = torch.Generator().manual_seed(10 + bits)
     codes = torch.randint(0, 2 ** bits, (2, 3, 4, 128), generator=g)
