@@ -21,12 +21,14 @@
 //     the workgroup instead runs an exact radix select over the whole row
 //     (11/11/10-bit digits), collects in index order and sorts the k results.
 // Step 3 also clears the histogram and list counters, which are zero between
-// calls.  Short rows, and selections larger than the lists hold (k > 8192),
-// run step 3's exact path alone; for k > 8192 it lists the selection by
+// calls.  Rows that one workgroup's registers hold are selected there in one
+// launch (up to 4096 elements by digit passes, up to 65536 by counting where
+// there are enough rows).  Other short rows, and selections larger than the
+// lists hold (k > 8192), run step 3's exact path alone; for k > 8192 it lists the selection by
 // ascending index, and a sorted output then takes two more launches: blocks
 // of 8192 selected entries sorted in LDS, then each entry's final slot from
 // its rank in its own block plus binary searches in the others.
-#include "wave_select.h"
+#include "row_select.h"
 
 namespace bytes_amd {
 
@@ -91,6 +93,15 @@ __device__ __forceinline__ void load4(__amdgpu_buffer_rsrc_t rs, int i, int n, u
   }
 #pragma unroll
   for (int j = 0; j < 4; ++j) ok[j] = i + j < n;
+}
+
+template <bool VEC>
+__device__ __forceinline__ f32x4 load4f(__amdgpu_buffer_rsrc_t rs, int i) {
+  if constexpr (VEC) return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, i * 4, 0, 0));
+  f32x4 v;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, (i + j) * 4, 0, 0));
+  return v;
 }
 
 __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m) {
@@ -631,85 +642,10 @@ __global__ __launch_bounds__(kTopkThreads) void topk_select_kernel(const float* 
   }
 }
 
-// ---- short rows: one wave per row ----
-// Many rows of at most kWaveRow elements with k <= kWaveK: the row's order keys
-// stay in the wave's registers (lane holds elements PER*lane .. +PER), the
-// three digit passes histogram them in the wave's LDS and pick the digit with
-// a suffix scan over the lanes, and the selection is compacted in index order
-// (unsorted) or into an LDS list that an in-wave bitonic sort orders by
-// (score desc, index asc).  No workgroup barrier anywhere.
-constexpr int kWaveRow = 4096;
-constexpr int kWaveK = 256;
-constexpr int kWaveRowsPerWG = 4;
-
-template <bool VEC, int PER>
-__global__ __launch_bounds__(64 * kWaveRowsPerWG) void topk_wave_kernel(const float* scores, int64_t row_stride,
-                                                                        int64_t rows, int n, int k, int32_t* out,
-                                                                        int64_t out_stride, int sorted,
-                                                                        uint32_t* ghist) {
-  static_assert(PER % 4 == 0 && 64 * PER <= kWaveRow, "keys per lane");
-  __shared__ __attribute__((aligned(16))) uint32_t hist_s[kWaveRowsPerWG][kBins];
-  __shared__ uint64_t sb_s[kWaveRowsPerWG][kWaveK];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int64_t row = (int64_t)blockIdx.x * kWaveRowsPerWG + w;
-  if (row >= rows) return;                       // wave-uniform
-  uint32_t* hist = hist_s[w];
-  uint64_t* sb = sb_s[w];
-  const float* x = scores + row * row_stride;
-  const auto rs = row_rsrc(x, n);
-  int32_t* o = out + row * out_stride;
-
-  uint32_t key[PER];
-  const int i0 = PER * lane;                     // this lane's first element
-#pragma unroll
-  for (int j = 0; j < PER / 4; ++j) {
-    uint32_t kq[4];
-    bool okq[4];
-    load4<VEC>(rs, i0 + 4 * j, n, kq, okq);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) key[4 * j + e] = kq[e];
-  }
-  uint32_t T, need;
-  wave_select_threshold<PER>(key, n, k, hist, T, need);
-  if (ghist) {                                   // a histogram the caller built: leave it at zero
-    u32x4* gh = reinterpret_cast<u32x4*>(ghist + row * kBins) + lane * 8;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) gh[q] = u32x4{0u, 0u, 0u, 0u};
-  }
-  // compaction in index order (lane, q): slot = selected keys before this one
-  wave_select_compact<PER>(key, n, T, need, [&](uint32_t pos, int idx, uint32_t kk) {
-    if (sorted) sb[pos] = sort_val(kk, idx);
-    else o[pos] = idx;
-  });
-  if (!sorted) return;
-
-  // in-wave bitonic sort of sb[0, P) into descending order (padding zeros sort last)
-  int P = 64;
-  while (P < k) P <<= 1;
-  for (int i = k + lane; i < P; i += 64) sb[i] = 0ull;
-  wave_lds_sync();
-  for (int size = 2; size <= P; size <<= 1) {
-    for (int stride = size >> 1; stride >= 1; stride >>= 1) {
-      for (int p = lane; p < P / 2; p += 64) {
-        const int lo = ((p & ~(stride - 1)) << 1) | (p & (stride - 1));
-        const int hi = lo + stride;
-        const bool desc = (lo & size) == 0;
-        const uint64_t va = sb[lo], vb = sb[hi];
-        if ((va < vb) == desc) {
-          sb[lo] = vb;
-          sb[hi] = va;
-        }
-      }
-      wave_lds_sync();
-    }
-  }
-  for (int i = lane; i < k; i += 64) o[i] = (int32_t)(0xFFFFFFFFu - (uint32_t)sb[i]);
-}
-
-// Rows of at most kSmallRow elements that the wave kernel does not take (few
-// rows, or larger k): one 256-thread workgroup per row, the row's order keys
-// in registers (thread t holds elements PER*t .. +PER, read from memory once),
-// selected by block_select (8-bit digit passes from the highest bit in which
+// ---- short rows ----
+// Rows of at most kSmallRow elements: one 256-thread workgroup per row, the
+// row's order keys in registers (thread t holds elements PER*t .. +PER, read
+// from memory once), selected by block_select (8-bit digit passes from the highest bit in which
 // the row's keys differ, one barrier per pass); one scan of the per-thread
 // counts places the selection in index order, or into an LDS list sorted by
 // (score desc, index asc).
@@ -760,6 +696,63 @@ __global__ __launch_bounds__(kSmallThreads) void topk_small_kernel(const float* 
   __syncthreads();
   bitonic_desc<NT>(sb, P);
   for (int i = tid; i < k; i += NT) o[i] = (int32_t)(0xFFFFFFFFu - (uint32_t)sb[i]);
+}
+
+// ---- a longer row in one workgroup's registers ----
+// Rows of up to 64 keys per thread are read once, kept as order keys in
+// registers and selected by counting (row_select.h); the selection is written
+// in index order, or (SORT, k <= kRowSortK) listed in LDS and sorted by
+// (score desc, index asc).  Bound by VALU (two operations per key and count,
+// five to six counts, four to make the key), then by the one read of the row.
+// us per call at 2048 rows, unsorted, here against the paths of the same
+// shapes without it (one 1024-thread workgroup re-reading the row for three
+// digit passes and the collection up to 16384, else histogram, filter and
+// select launches): n = 8192 k = 410 31 / 91, 16384 k = 819 51 / 154, 32768
+// k = 1638 95 / 196, 65536 k = 655 194 / 287.
+constexpr int kRowSortK = 1024;
+constexpr int kRowMax = 65536;         // 1024 threads x 64 keys
+
+template <bool VEC, int NT, int PER, bool SORT>
+__global__ __launch_bounds__(NT, PER == 64 ? 4 : 6) void topk_row_kernel(const float* scores, int64_t row_stride,
+                                                                         int n, int k, int32_t* out,
+                                                                         int64_t out_stride, uint32_t* ghist) {
+  __shared__ __attribute__((aligned(16))) RowLds<NT, PER> lds;
+  __shared__ uint64_t sb[SORT ? kRowSortK : 1];
+  const int t = threadIdx.x;
+  const int64_t row = blockIdx.x;
+  const float* x = scores + row * row_stride;
+  const auto rs = row_rsrc(x, n);
+  int32_t* o = out + row * out_stride;
+  uint32_t key[PER];
+  row_load<NT, PER>(key, n, [&](int r) { return load4f<VEC>(rs, (r * NT + t) * 4); });
+  const RowSel s = row_search<NT, PER>(key, n, (uint32_t)k, lds);
+  if (ghist) {                                   // a histogram the caller built: leave it at zero
+    u32x4* gh = reinterpret_cast<u32x4*>(ghist + row * kBins);
+    for (int q = t; q < kBins / 4; q += NT) gh[q] = u32x4{0u, 0u, 0u, 0u};
+  }
+  if constexpr (!SORT) {
+    row_emit<NT, PER>(key, s, lds, [&](uint32_t pos, int idx) { o[pos] = idx; });
+  } else {
+    int P = 64;
+    while (P < k) P <<= 1;
+    for (int i = k + t; i < P; i += NT) sb[i] = 0ull;   // padding sorts last
+    row_emit<NT, PER>(key, s, lds, [&](uint32_t pos, int idx) { sb[pos] = sort_val(order_key(x[idx]), idx); });
+    __syncthreads();
+    bitonic_desc<NT>(sb, P);
+    for (int i = t; i < k; i += NT) o[i] = (int32_t)(0xFFFFFFFFu - (uint32_t)sb[i]);
+  }
+}
+
+template <bool VEC, int NT, int PER>
+static void topk_row_launch(const float* scores, int64_t rows, int n, int64_t row_stride, int k, int32_t* out,
+                            int64_t out_stride, int sorted, uint32_t* gh, hipStream_t st) {
+  const dim3 grid((unsigned)rows), block(NT);
+  if (sorted)
+    hipLaunchKernelGGL((topk_row_kernel<VEC, NT, PER, true>), grid, block, 0, st, scores, row_stride, n, k, out,
+                       out_stride, gh);
+  else
+    hipLaunchKernelGGL((topk_row_kernel<VEC, NT, PER, false>), grid, block, 0, st, scores, row_stride, n, k, out,
+                       out_stride, gh);
 }
 
 // ---- k > kTopkMaxK on long rows: the selection in index order ----
@@ -1066,23 +1059,7 @@ static int topk_launch(const float* scores, int64_t rows, int n, int64_t row_str
     lds_set = true;
   }
   const int parts = (n + kSlice - 1) / kSlice;
-  // one wave per row when there are more rows than CUs: the one-workgroup
-  // path (16 waves per row, one workgroup per CU at a time) then runs in
-  // several generations, while four rows per workgroup all stay resident;
-  // with fewer rows the 16-wave workgroups finish each row sooner
-  if (n <= kWaveRow && k <= kWaveK && rows > device_cu_count()) {
-    const int64_t g = (rows + kWaveRowsPerWG - 1) / kWaveRowsPerWG;
-    if (g > 0x7FFFFFFFL) return (int)hipErrorInvalidConfiguration;
-    uint32_t* gh = hist_ready ? ws.hist : nullptr;
-    if (n <= 2048)
-      hipLaunchKernelGGL((topk_wave_kernel<VEC, 32>), dim3((unsigned)g), dim3(64 * kWaveRowsPerWG), 0, st, scores,
-                         row_stride, rows, n, k, out, out_stride, sorted, gh);
-    else
-      hipLaunchKernelGGL((topk_wave_kernel<VEC, 64>), dim3((unsigned)g), dim3(64 * kWaveRowsPerWG), 0, st, scores,
-                         row_stride, rows, n, k, out, out_stride, sorted, gh);
-    return (int)hipGetLastError();
-  }
-  // other rows of at most kSmallRow elements: a 256-thread workgroup per row
+  // rows of at most kSmallRow elements: a 256-thread workgroup per row
   if (n <= kSmallRow && (!sorted || k <= kSmallSortK)) {
     if (rows > 0x7FFFFFFFL) return (int)hipErrorInvalidConfiguration;
     uint32_t* gh = hist_ready ? ws.hist : nullptr;
@@ -1096,6 +1073,24 @@ static int topk_launch(const float* scores, int64_t rows, int n, int64_t row_str
     else
       hipLaunchKernelGGL((topk_small_kernel<VEC, 16>), grid, block, 0, st, scores, row_stride, n, k, out,
                          out_stride, sorted, gh);
+    return (int)hipGetLastError();
+  }
+  // longer rows that one workgroup's registers hold, where the rows alone keep
+  // the chip busy; fewer rows finish sooner on 16 waves a row (up to 8192
+  // elements: 64 rows of 5000 11.7 us there against 13.9, 2048 rows of 8192
+  // 91 against 31) or spread over several workgroups a row (above 16384: 128
+  // rows of 65536 32.5 against 37.6, 256 rows 49.5 against 41.9; sorted, 300
+  // rows 65 against 72).  Rows of 8193 to 16384 gain at any count (4 rows of
+  // 16384: 19.3 against 13.6).
+  const int cus = device_cu_count();
+  const bool row_regs = n <= 8192 ? rows > cus : n <= kShortRow ? true : n <= kRowMax && rows >= (sorted ? 2 : 1) * cus;
+  if (row_regs && (!sorted || k <= kRowSortK)) {
+    if (rows > 0x7FFFFFFFL) return (int)hipErrorInvalidConfiguration;
+    uint32_t* gh = hist_ready ? ws.hist : nullptr;
+    if (n <= 8192) topk_row_launch<VEC, 256, 32>(scores, rows, n, row_stride, k, out, out_stride, sorted, gh, st);
+    else if (n <= 16384) topk_row_launch<VEC, 512, 32>(scores, rows, n, row_stride, k, out, out_stride, sorted, gh, st);
+    else if (n <= 32768) topk_row_launch<VEC, 512, 64>(scores, rows, n, row_stride, k, out, out_stride, sorted, gh, st);
+    else topk_row_launch<VEC, 1024, 64>(scores, rows, n, row_stride, k, out, out_stride, sorted, gh, st);
     return (int)hipGetLastError();
   }
   // k beyond the list capacity on long rows: filter, per-row select, ordered write

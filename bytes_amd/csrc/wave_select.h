@@ -1,19 +1,12 @@
-// Exact top-k selection over a short row by one wave or by one workgroup
-// (used by the top-k kernels and by kernels that select inside their
-// prologue).
+// Exact top-k selection over a short row by one workgroup (used by the top-k
+// kernels and by kernels that select inside their prologue).
 //
-// The row's n <= 64 * PER order keys (score_order_key) sit in the wave's
-// registers, lane l holding elements PER*l .. PER*l + PER - 1.  The selection
-// is the top k under one total order: key descending, index ascending on
-// equal keys.  wave_select_threshold finds the k-th largest key T and how
-// many keys equal to T are taken (the lowest-indexed ones): digit passes of
-// 11 bits start at the highest bit in which the row's keys differ, histogram
-// the keys matching the prefix so far in the wave's LDS (kBins words) and
-// pick the digit from a suffix scan over the lanes.  wave_select_compact then
-// lists the selected indices in ascending index order.  Wave-level
-// synchronisation only: no workgroup barrier.
-// block_select / block_select_emit do the same with the NT threads of a
-// workgroup, thread t holding elements PER*t .. +PER (described below).
+// The row's n <= NT * PER order keys (score_order_key) sit in registers,
+// thread t holding elements PER*t .. PER*t + PER - 1.  The selection is the
+// top k under one total order: key descending, index ascending on equal keys.
+// block_select finds the k-th largest key by digit passes over LDS
+// histograms, block_select_emit lists the selected indices in ascending
+// order.
 #pragma once
 #include "common.h"
 
@@ -21,116 +14,10 @@ namespace bytes_amd {
 
 constexpr int kBins = 2048;            // digit = 11 bits of the order key
 
-__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v, int lane) { return wave_prefix_sum(v); }
-
 // Inclusive suffix sum over the 64 lanes (lane i: sum over lanes >= i).
 __device__ __forceinline__ uint32_t wave_suffix_sum(uint32_t v) {
   const uint32_t incl = wave_prefix_sum(v);
   return (uint32_t)__builtin_amdgcn_readlane((int)incl, 63) - incl + v;
-}
-
-template <int PER>
-__device__ __forceinline__ void wave_select_threshold(const uint32_t (&key)[PER], int n, int k, uint32_t* hist,
-                                                      uint32_t& T, uint32_t& need) {
-  const int lane = threadIdx.x & 63;
-  const int i0 = PER * lane;
-  auto valid = [&](int q) { return i0 + q < n; };
-  uint32_t kmin = 0xFFFFFFFFu, kmax = 0u;
-#pragma unroll
-  for (int q = 0; q < PER; ++q)
-    if (valid(q)) {
-      kmin = min(kmin, key[q]);
-      kmax = max(kmax, key[q]);
-    }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    kmin = min(kmin, (uint32_t)__shfl_xor((int)kmin, off, 64));
-    kmax = max(kmax, (uint32_t)__shfl_xor((int)kmax, off, 64));
-  }
-  const uint32_t diff = kmin ^ kmax;
-  const int hb = diff ? 31 - __builtin_clz(diff) : -1;
-  uint32_t pmask = hb < 0 ? 0xFFFFFFFFu : ~(uint32_t)((2ull << hb) - 1ull);
-  uint32_t prefix = kmin & pmask, kr = (uint32_t)k;
-#pragma unroll 1
-  for (int hi = hb; hi >= 0; hi -= 11) {
-    const int shift = hi >= 10 ? hi - 10 : 0;
-    const uint32_t dmask = (1u << (hi - shift + 1)) - 1u;
-    u32x4* h4 = reinterpret_cast<u32x4*>(hist) + lane * 8;      // this lane's 32 bins
-#pragma unroll
-    for (int q = 0; q < 8; ++q) h4[q] = u32x4{0u, 0u, 0u, 0u};
-    wave_lds_sync();
-#pragma unroll
-    for (int q = 0; q < PER; ++q)
-      if (valid(q) && (key[q] & pmask) == prefix) atomicAdd(&hist[(key[q] >> shift) & dmask], 1u);
-    wave_lds_sync();
-    uint32_t c[32];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const u32x4 v = h4[q];
-      c[4 * q] = v[0]; c[4 * q + 1] = v[1]; c[4 * q + 2] = v[2]; c[4 * q + 3] = v[3];
-    }
-    uint32_t s = 0;
-#pragma unroll
-    for (int b = 0; b < 32; ++b) s += c[b];
-    // inclusive suffix sum over lanes (bins above this lane's range included)
-    const uint32_t suf = wave_suffix_sum(s);
-    const uint32_t above_lane = suf - s;         // keys in digits above this lane's bins
-    // digit d: count(digits > d) < kr <= count(digits >= d)
-    const bool mine = above_lane < kr && kr <= suf;
-    uint32_t acc = above_lane, d = 0u, above = 0u;
-    bool got = false;
-#pragma unroll
-    for (int b = 31; b >= 0; --b) {
-      if (!got && acc + c[b] >= kr) {
-        got = true;
-        d = 32u * lane + b;
-        above = acc;
-      }
-      acc += c[b];
-    }
-    const int src = __ffsll((unsigned long long)__ballot(mine)) - 1;
-    d = (uint32_t)__builtin_amdgcn_readlane((int)d, src);
-    above = (uint32_t)__builtin_amdgcn_readlane((int)above, src);
-    kr -= above;
-    prefix |= d << shift;
-    pmask |= dmask << shift;
-    wave_lds_sync();
-  }
-  T = prefix;
-  need = kr;                                     // keys equal to T to take (>= 1)
-}
-
-// Selected indices in ascending order: out[slot] for slot < k, through
-// emit(slot, index, key).
-template <int PER, class EMIT>
-__device__ __forceinline__ void wave_select_compact(const uint32_t (&key)[PER], int n, uint32_t T, uint32_t need,
-                                                    EMIT emit) {
-  const int lane = threadIdx.x & 63;
-  const int i0 = PER * lane;
-  auto valid = [&](int q) { return i0 + q < n; };
-  uint32_t ne = 0u, ng = 0u;
-#pragma unroll
-  for (int q = 0; q < PER; ++q) {
-    ne += (valid(q) && key[q] == T) ? 1u : 0u;
-    ng += (valid(q) && key[q] > T) ? 1u : 0u;
-  }
-  uint32_t rank = wave_incl_scan(ne, lane) - ne;          // keys equal to T before this lane
-  const uint32_t take_eq = rank >= need ? 0u : (need - rank < ne ? need - rank : ne);
-  const uint32_t nt = ng + take_eq;
-  uint32_t pos = wave_incl_scan(nt, lane) - nt;
-#pragma unroll
-  for (int q = 0; q < PER; ++q) {
-    const bool v = valid(q);
-    bool take = v && key[q] > T;
-    if (v && key[q] == T) {
-      take = rank < need;
-      ++rank;
-    }
-    if (take) {
-      emit(pos, i0 + q, key[q]);
-      ++pos;
-    }
-  }
 }
 
 // ---- workgroup selection ----

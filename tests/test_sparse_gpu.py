@@ -179,8 +179,7 @@ def test_topk_large_k_row_batches(dev):
 @pytest.mark.parametrize("rows,n,k", [(600, 2048, 128), (600, 1000, 1), (300, 4096, 256), (700, 2051, 17),
                                       (260, 64, 64), (1000, 4095, 200)])
 def test_topk_many_short_rows(dev, rows, n, k, sorted_out):
-    """More rows than CUs with n <= 4096 and k <= 256: the one-wave-per-row
-    selection (ties, +-0, NaN, +-inf and all-equal rows included)."""
+    """More rows than CUs with n <= 4096 and k <= 256 (ties, +-0, NaN, +-inf and all-equal rows included)."""
     s = _tie_heavy(rows, n, seed=n + k + rows)
     s[2] = 0.5                                             # an all-equal row
     s[3, : n // 2] = float("inf")                          # more infinities than k
@@ -191,8 +190,7 @@ def test_topk_many_short_rows(dev, rows, n, k, sorted_out):
 @pytest.mark.parametrize("rows,n,k", [(1, 1, 1), (1, 3, 2), (5, 64, 64), (28, 2048, 1024), (3, 4096, 4096),
                                       (4, 4096, 1024), (2, 3000, 2000), (280, 1500, 512), (7, 4095, 1)])
 def test_topk_small_rows(dev, rows, n, k):
-    """Rows of at most 4096 elements outside the one-wave path: one 256-thread
-    workgroup per row (sorted output up to k = 1024; larger sorted k takes the
+    """Rows of at most 4096 elements: one 256-thread workgroup per row (sorted output up to k = 1024; larger sorted k takes the
     whole-row sort)."""
     s = _tie_heavy(rows, n, seed=3 * n + k)
     if rows > 3:
@@ -225,8 +223,8 @@ def test_topk_small_rows_continuous(dev, rows, n, k, shift):
 @pytest.mark.parametrize("rows,n,k", [(300, 2048, 128), (28, 2048, 128), (280, 4096, 600), (5, 1000, 17)])
 def test_topk_narrow_range_rows(dev, rows, n, k):
     """Scores in a narrow range (every key shares its top bits; the digit
-    passes start below them), with exact ties and an all-equal row, on the
-    one-wave path (more rows than CUs, k <= 256) and the workgroup path."""
+    passes start below them), with exact ties and an all-equal row, for more
+    and fewer rows than CUs."""
     g = torch.Generator().manual_seed(rows + n + k)
     s = 3.0 + torch.rand(rows, n, generator=g) * 0.5
     s[0, 10:40] = 3.25                                       # a block of exact ties
@@ -236,6 +234,38 @@ def test_topk_narrow_range_rows(dev, rows, n, k):
     for so in (True, False):
         got = SP.topk_indices(s.to(dev), k, sorted=so).cpu()
         assert torch.equal(got.long(), R.topk_indices(s, k, sorted_by_score=so)), so
+
+
+@pytest.mark.parametrize("rows,n,k", [(257, 4097, 40), (300, 8191, 8191), (3, 8193, 1), (5, 16384, 819),
+                                      (256, 16385, 1000), (256, 32768, 3000), (513, 16500, 1024),
+                                      (512, 40001, 200), (256, 65536, 9000)])
+def test_topk_rows_selected_by_counting(dev, rows, n, k):
+    """Rows of 4097 to 65536 elements held in one workgroup's registers (sorted
+    up to k = 1024): continuous scores, the same shifted and narrowed, ties
+    and lattices, half the row -inf or +inf, NaN of both signs, one value in
+    the whole row, one value far above the others, and rows that start off
+    16-byte boundaries."""
+    g = torch.Generator().manual_seed(n + k)
+    s = torch.randn(rows, n, generator=g)
+    m = min(rows, 256)
+    s[: m // 4 * 4].reshape(4, -1, n)[1] *= 1e-3
+    s[: m // 4 * 4].reshape(4, -1, n)[1] += 40.0
+    s[: m // 4 * 4].reshape(4, -1, n)[2] = s[: m // 4 * 4].reshape(4, -1, n)[2].mul(8).round() / 8
+    for i, f in enumerate([lambda r: r.fill_(-2.5), lambda r: r[: n // 2].fill_(float("-inf")),
+                           lambda r: r[n // 3:].fill_(float("inf")), lambda r: r[::7].fill_(float("nan"))]):
+        if i + 1 < rows:
+            f(s[i + 1])
+    if rows > 8:
+        s[5, 3] = -float("nan")
+        s[6, n - 1] = 3e38
+        s[7] = torch.where(torch.arange(n) % 3 == 0, 0.0, -0.0)
+        s[8] = torch.arange(n).float()
+    want = {so: R.topk_indices(s, k, sorted_by_score=so) for so in ((True, False) if k <= 1024 else (False,))}
+    for so, w in want.items():
+        assert torch.equal(SP.topk_indices(s.to(dev), k, sorted=so).cpu().long(), w), so
+    big = torch.zeros(rows * n + 1, device=dev)
+    big[1:] = s.reshape(-1).to(dev)
+    assert torch.equal(SP.topk_indices(big[1:].reshape(rows, n), k, sorted=False).cpu().long(), want[False])
 
 
 def test_topk_many_short_rows_unaligned(dev):
