@@ -131,6 +131,10 @@ SIGNATURES: Dict[str, Tuple] = {
     "bytes_select_mask_at": (c_vp, c_i64, c_int, c_i64, c_i64, c_vp, c_int, c_int, c_int, c_vp),
     "bytes_select_merge": (c_vp, c_i64, c_int, c_int, c_vp, c_i64, c_vp, c_i64, c_int, c_int, c_int, c_i64, c_vp,
                            c_i64, c_int, c_vp, c_i64, c_int, c_vp),
+    "bytes_select_step": (
+        c_vp, c_i64, c_int, c_int, c_int,                       # cand, row stride, off, nrun, chunk keys
+        c_vp, c_i64, c_int, c_vp, c_int, c_int, c_int, c_int,   # ridx, row stride, kc0, pos, Qc, local_w, S, kb
+        c_i64, c_vp, c_i64, c_int, c_vp, c_i64, c_vp, c_vp),    # rows, next scores, indices, final indices, stream
     "bytes_select_recent": (c_vp, c_int, c_i64, c_int, c_vp, c_vp),
 }
 _RESTYPES = {"bytes_error_string": ctypes.c_char_p}

@@ -13,10 +13,10 @@
 // no LDS traffic but one word per wave.  The search keeps a bracket [lo, hi]
 // with count(>= lo) >= k > count(> hi).  The first trial comes from a sample
 // (the first wave's first keys, searched in that wave alone), the second lies
-// past the k-th key by the sample's density, and from then on the trial
-// interpolates between the bracket's counts in the value domain; where that
-// shrank the bracket by less than half it takes the middle value, and from
-// the twelfth count on the middle key, so at most 44 counts are ever needed
+// past the k-th key by the sample's spacing, and from then on the trial
+// interpolates between the bracket's counts in key space; where that shrank
+// the bracket by less than half it takes the middle key, and so does every
+// trial from the twelfth count on, so at most 44 counts are ever needed
 // (five or six on ordinary scores, about 30 where most scores are equal to
 // others).  The selection's membership masks are then taken by wave ballots,
 // and each thread lists its PER consecutive elements from them, so the output
@@ -47,10 +47,9 @@ __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t x) {   // every lane's
   return (uint32_t)__builtin_amdgcn_readlane((int)wave_prefix_sum(x), 63);
 }
 
-// Sum over the NT threads; `turn` alternates between calls.
+// Sum of the waves' totals; `turn` alternates between calls.
 template <int NT, class L>
-__device__ __forceinline__ uint32_t row_sum(uint32_t x, L& lds, int& turn) {
-  const uint32_t s = wave_sum_u32(x);
+__device__ __forceinline__ uint32_t row_sum(uint32_t s, L& lds, int& turn) {
   if constexpr (NT == 64) return s;
   constexpr int NW = NT / 64;
   turn ^= 1;
@@ -62,16 +61,15 @@ __device__ __forceinline__ uint32_t row_sum(uint32_t x, L& lds, int& turn) {
   return (uint32_t)__builtin_amdgcn_readfirstlane((int)t);
 }
 
+// Keys at or above t among the wave's N per lane.  (Counting some or all of
+// them on the scalar unit, as population counts of the compare's lane mask, is
+// 5% slower.)
 template <int N>
-__device__ __forceinline__ uint32_t count_ge(const uint32_t* key, uint32_t t) {
+__device__ __forceinline__ uint32_t wave_count_ge(const uint32_t* key, uint32_t t) {
   uint32_t c = 0u;
 #pragma unroll
   for (int q = 0; q < N; ++q) c += key[q] >= t ? 1u : 0u;
-  return c;
-}
-
-__device__ __forceinline__ float order_key_value(uint32_t k) {   // inverse of score_order_key
-  return __uint_as_float(k ^ (~(uint32_t)((int)k >> 31) | 0x80000000u));
+  return wave_sum_u32(c);
 }
 
 // The order key of a score that is not NaN (a NaN's key, of either sign,
@@ -87,17 +85,15 @@ struct RowBracket {
   bool slow;                           // the last interpolation shrank the bracket by less than half
 };
 
-// A trial key in (lo, hi] (lo < hi).  Every value here is the same on every
-// lane; the arithmetic needs no accuracy.
-__device__ __forceinline__ uint32_t row_trial(const RowBracket& b, uint32_t k, bool middle_key) {
-  const uint32_t mid = b.lo + ((b.hi - b.lo + 1u) >> 1);
-  const float xl = order_key_value(b.lo), xh = order_key_value(b.hi);
-  const float f = b.slow ? 0.5f
-                         : ((float)(b.cl - k) + 0.5f) * __builtin_amdgcn_rcpf((float)(b.cl - b.ch));
-  const float x = __builtin_fmaf(xh - xl, f, xl);   // infinite or NaN where an end is
-  const bool fin = fabsf(x) < __builtin_inff() && !middle_key;
-  const uint32_t t = min(max(order_key_ordinary(x), b.lo + 1u), b.hi);
-  return (uint32_t)__builtin_amdgcn_readfirstlane((int)(fin ? t : mid));
+// A trial key in (lo, hi] (lo < hi): where a line through the bracket's counts
+// reaches k, in key space (which is linear in the score within a binade); the
+// middle key where the last such line did badly.  Every value here is the same
+// on every lane; the arithmetic needs no accuracy.
+__device__ __forceinline__ uint32_t row_trial(const RowBracket& b, uint32_t k, bool middle) {
+  const float f = ((float)(b.cl - k) + 0.5f) * __builtin_amdgcn_rcpf((float)(b.cl - b.ch));
+  const uint32_t w = b.hi - b.lo;
+  const uint32_t d = middle || b.slow ? (w >> 1) + 1u : (uint32_t)(f * (float)w);
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)(b.lo + min(max(d, 1u), w)));
 }
 
 // One count's consequence; true once the k-th key is known (b.lo).
@@ -121,10 +117,10 @@ struct RowSel {
   bool all;
 };
 
-// First trial and density (keys per unit of score) from a sample of one wave's
-// keys: the sample's value of the k-th rank.
+// First trial, and how far one rank is from the next in key space, from a
+// sample of one wave's keys: the sample's value of the k-th rank.
 template <int N>
-__device__ __forceinline__ void row_sample(const uint32_t* key, int n, uint32_t k, uint32_t& t, float& dens) {
+__device__ __forceinline__ void row_sample(const uint32_t* key, int n, uint32_t k, uint32_t& t, float& gap) {
   uint32_t mn = 0xFFFFFFFFu, mx = 0u, ns = 0u;
 #pragma unroll
   for (int q = 0; q < N; ++q) {
@@ -134,23 +130,22 @@ __device__ __forceinline__ void row_sample(const uint32_t* key, int n, uint32_t 
   }
   wave_minmax_u32(mn, mx);
   ns = wave_sum_u32(ns);
-  const float rate = (float)n * __builtin_amdgcn_rcpf((float)ns);   // keys per sampled key
-  const uint32_t ks = max((uint32_t)((float)k * __builtin_amdgcn_rcpf(rate)), 1u);
+  const float part = (float)ns * __builtin_amdgcn_rcpf((float)n);   // of the row's keys
+  const uint32_t ks = max((uint32_t)((float)k * part), 1u);
   RowBracket b;
   b.lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(mn + 1u));
   b.hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)mx);
   b.cl = ns;
   b.ch = 0u;
   b.slow = false;
-  // narrow until the bracket holds about two standard errors of the rank
+  // narrow until the bracket holds about one standard error of the rank
   const uint32_t cap = 2u + (uint32_t)__builtin_amdgcn_sqrtf((float)ks);
-  for (int i = 0; i < 8 && b.lo < b.hi && b.cl - b.ch > cap && b.cl != ks; ++i) {
+  for (int i = 0; i < 10 && b.lo < b.hi && b.cl - b.ch > cap && b.cl != ks; ++i) {
     const uint32_t u = row_trial(b, ks, false);
-    row_update(b, u, wave_sum_u32(count_ge<N>(key, u)), ks);
+    row_update(b, u, wave_count_ge<N>(key, u), ks);
   }
   t = b.lo < b.hi && b.cl != ks ? row_trial(b, ks, false) : b.lo;
-  const float width = order_key_value(b.hi) - order_key_value(b.lo);
-  dens = (float)(b.cl - b.ch) * rate * __builtin_amdgcn_rcpf(width);   // may be anything where ties or infinities abound
+  gap = (float)(b.hi - b.lo) * part * __builtin_amdgcn_rcpf((float)(b.cl - b.ch));
 }
 
 // k-th largest of the row's keys.  Every thread calls it; n >= k >= 1.
@@ -159,35 +154,33 @@ __device__ __forceinline__ RowSel row_search(const uint32_t (&key)[PER], int n, 
   constexpr int NS = PER < 16 ? PER : 16;        // sampled keys per lane
   int turn = 0;
   uint32_t t;
-  float dens;
+  float gap;
   if constexpr (NT == 64) {
-    row_sample<NS>(key, n, k, t, dens);
+    row_sample<NS>(key, n, k, t, gap);
   } else {
     if (threadIdx.x < 64) {
-      row_sample<NS>(key, n, k, t, dens);
+      row_sample<NS>(key, n, k, t, gap);
       if (threadIdx.x == 0) {
         lds.guess[0] = t;
-        lds.guess[1] = __float_as_uint(dens);
+        lds.guess[1] = __float_as_uint(gap);
       }
     }
     __syncthreads();
     t = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds.guess[0]);
-    dens = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)lds.guess[1]));
+    gap = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)lds.guess[1]));
   }
   RowBracket b{1u, 0xFFFFFFFFu, (uint32_t)n, 0u, false};
   if ((uint32_t)n > k) {
-    float reach = 1.5f;
+    gap *= 1.5f;
     for (int i = 0;; ++i) {
-      if (row_update(b, t, row_sum<NT>(count_ge<PER>(key, t), lds, turn), k)) break;
+      if (row_update(b, t, row_sum<NT>(wave_count_ge<PER>(key, t), lds, turn), k)) break;
       if (i < 4 && (b.lo == 1u || b.hi == 0xFFFFFFFFu)) {
-        // one side only so far: past the k-th key by the sample's density
+        // one side only so far: past the k-th key by the sample's spacing
         const bool up = b.hi == 0xFFFFFFFFu;
-        const uint32_t miss = up ? b.cl - k : k - b.ch;
-        const float step = ((float)miss * reach + 2.f) * __builtin_amdgcn_rcpf(dens);
-        const float x = order_key_value(up ? b.lo : b.hi) + (up ? step : -step);
-        reach *= 4.f;
-        const uint32_t u = fabsf(x) < __builtin_inff() ? order_key_ordinary(x) : b.lo + ((b.hi - b.lo + 1u) >> 1);
-        t = (uint32_t)__builtin_amdgcn_readfirstlane((int)min(max(u, b.lo + 1u), b.hi));
+        const float step = ((float)(up ? b.cl - k : k - b.ch) + 2.f) * gap;
+        const uint32_t w = b.hi - b.lo, d = max((uint32_t)fminf(step, (float)(w >> 1)), 1u);
+        t = (uint32_t)__builtin_amdgcn_readfirstlane((int)(up ? b.lo + d : b.hi - d + 1u));
+        gap *= 4.f;
         b.slow = false;
       } else {
         t = row_trial(b, k, i >= 11);
@@ -210,15 +203,15 @@ __device__ __forceinline__ void row_load(uint32_t (&key)[PER], int n, LOAD load)
   f32x4 raw[PER / 4];
 #pragma unroll
   for (int r = 0; r < PER / 4; ++r) raw[r] = load(r);
-  bool odd = false;
+  float nan = 0.f;                               // IEEE maximum: NaN as soon as one value is
 #pragma unroll
   for (int r = 0; r < PER / 4; ++r)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       key[4 * r + e] = order_key_ordinary(raw[r][e]);
-      odd = odd || raw[r][e] != raw[r][e];
+      nan = __builtin_elementwise_maximum(nan, raw[r][e]);
     }
-  if (__ballot(odd))
+  if (__ballot(nan != nan))
 #pragma unroll
     for (int q = 0; q < PER; ++q)
       if (key[q] - kKeyNegInf > kKeyPosInf - kKeyNegInf) key[q] = 0xFFFFFFFFu;

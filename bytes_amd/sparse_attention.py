@@ -97,19 +97,23 @@ def _fill(idx: torch.Tensor, pos: torch.Tensor, Qc: int, S: int, k_out: int, dty
     return out.reshape(*idx.shape[:-1], k_out)
 
 
+STEP_ROW, STEP_SORT = 16384, 2048   # candidates (and, after the last chunk, selected ones) a fused step holds
+
+
 def _stream_select(qf, sel_keys, pos, Qc: int, S: int, kb: int, k_chunk: int, scaling: float, max_key: int,
                    local_w: int) -> torch.Tensor:
     """The streaming top-k of benchmarks/sparse_attention.py:286-309 over folded
-    rows qf [B, Hq*Qc, 1, D]: int32 key indices [B*Hq*Qc, kb] ordered by
-    (score desc, index asc), fillers (-inf, S) where a row has fewer than kb
-    candidates.
+    rows qf [B, Hq*Qc, 1, D]: int64 key indices [B*Hq*Qc, kb] ordered by
+    (score desc, index asc), S where a row has fewer than kb causal keys.
 
-    Each chunk of k_chunk keys is scored into cand[:, kbp:], masked (causal,
-    recent window) with its key offset, and the top kb of the row's running
-    list (cand[:, kbp - kb:kbp]) plus the chunk become the next running list,
-    written to the other buffer.  The running list comes first in each row, so
-    the top-k's lowest-position tie rule keeps the lowest key index on equal
-    scores; the last merge orders the list by score."""
+    Each chunk of k_chunk keys is scored into cand[:, kbp:]; the top kb of the
+    row's running list (cand[:, kbp - kb:kbp]) plus the chunk, masked (causal,
+    recent window) with its key offset, become the next running list, written
+    to the other buffer.  The running list comes first in each row, so the
+    top-k's lowest-position tie rule keeps the lowest key index on equal
+    scores; the last merge orders the list by score.  A step whose candidates
+    fit a workgroup's registers is one launch (bytes_select_step); others mask,
+    select and merge in launches of their own."""
     B, R1 = qf.shape[0], qf.shape[1]
     rows = B * R1
     dev = qf.device
@@ -127,15 +131,22 @@ def _stream_select(qf, sel_keys, pos, Qc: int, S: int, kb: int, k_chunk: int, sc
         buf = cand[cur]
         _score(qf, sel_keys[:, :, kc0:kc1], scaling, group_sum=False,
                out=buf.view(B, R1, W)[:, :, kbp:kbp + n])
-        call("bytes_select_mask_at", ptr(buf) + 4 * kbp, rows, n, W, kc0, ptr(pos), Qc, 1, int(local_w), st)
         off = kbp - nrun
         ksel = min(kb, nrun + n)
-        sel = _topk(buf[:, off:off + nrun + n], ksel, sorted=last)
         nxt = 1 - cur
-        call("bytes_select_merge", ptr(buf), W, off, nrun, ptr(ridx[cur]), kb, ptr(sel), sel.stride(0), ksel, kc0,
-             int(S), rows, None if last else ptr(cand[nxt]), W, kbp - kb, ptr(ridx[nxt]), kb, kb, st)
+        if (off & 3) + nrun + n <= STEP_ROW and not (last and ksel > STEP_SORT):
+            out = torch.empty((rows, kb), dtype=torch.int64, device=dev) if last else None
+            call("bytes_select_step", ptr(buf), W, off, nrun, n, ptr(ridx[cur]), kb, kc0, ptr(pos), Qc, int(local_w),
+                 int(S), kb, rows, ptr(cand[nxt]), W, kbp - kb, ptr(ridx[nxt]), kb, ptr(out) if last else None, st)
+            if last:
+                return out
+        else:
+            call("bytes_select_mask_at", ptr(buf) + 4 * kbp, rows, n, W, kc0, ptr(pos), Qc, 1, int(local_w), st)
+            sel = _topk(buf[:, off:off + nrun + n], ksel, sorted=last)
+            call("bytes_select_merge", ptr(buf), W, off, nrun, ptr(ridx[cur]), kb, ptr(sel), sel.stride(0), ksel,
+                 kc0, int(S), rows, None if last else ptr(cand[nxt]), W, kbp - kb, ptr(ridx[nxt]), kb, kb, st)
         cur, nrun = nxt, kb
-    return ridx[cur]
+    return _fill(ridx[cur], pos, Qc, S, kb, torch.int64)
 
 
 def select_topk(selector, q_blk, sel_keys, q_pos, S, kb, k_chunk, scaling, page=16, generator=None, local_w=0):
@@ -168,8 +179,8 @@ def select_topk(selector, q_blk, sel_keys, q_pos, S, kb, k_chunk, scaling, page=
         call("bytes_select_recent", ptr(pos), Qc, B * Hq * Qc, kb, ptr(out), stream_of(q_blk))
         return out
     max_key = min(pmax + 1, int(S), sel_keys.shape[2])
-    sel = _stream_select(qf, sel_keys, pos, Qc, int(S), kb, int(k_chunk), scaling, max_key, local_w)
-    return _fill(sel, pos, Qc, S, kb, torch.int64).reshape(B, Hq, Qc, kb)
+    return _stream_select(qf, sel_keys, pos, Qc, int(S), kb, int(k_chunk), scaling, max_key,
+                          local_w).reshape(B, Hq, Qc, kb)
 
 
 def _quest_select(q_blk, k_r, pos, S, kb, page, scaling, local_w=0):

@@ -296,6 +296,15 @@ int bytes_quest_gather_attn(const void* q, const void* k, const void* v, int kv_
  *   out_vals[r][out_off + i] (if out_vals is not NULL) and out_idx[r][i] =
  *   (score, key index) of candidate sel[r][i] for i < ksel, (-inf, S) for
  *   ksel <= i < kout.
+ * bytes_select_step: bytes_select_mask_at over the chunk, bytes_topk over the
+ *   row's candidates (the ksel = min(kb, nrun + n) best, by ascending position)
+ *   and bytes_select_merge with kout = kb, in one launch; the chunk's scores
+ *   stay unmasked in cand.  final_idx not NULL: the last step instead, which
+ *   writes final_idx [rows, kb] int64, the key indices ordered by score
+ *   (descending, lowest position first) as bytes_select_fill leaves them.
+ *   cand and cand_rs on 16-byte boundaries; (off & 3) + nrun + n <= 16384 and,
+ *   on the last step, ksel <= 2048 (hipErrorNotSupported above: the four calls
+ *   take any size).
  * bytes_select_recent: the "recent" selector (:261-265): out[r, j] =
  *   max(pos[r % Qc] - j, 0) int64 [rows, kb].
  * ------------------------------------------------------------------------- */
@@ -307,6 +316,10 @@ int bytes_select_merge(const void* cand, int64_t cand_rs, int off, int nrun, con
                        const void* sel, int64_t sel_rs, int ksel, int kc0, int S, int64_t rows, void* out_vals,
                        int64_t out_vals_rs, int out_off, void* out_idx, int64_t out_idx_rs, int kout,
                        void* stream);
+int bytes_select_step(const void* cand, int64_t cand_rs, int off, int nrun, int n, const void* ridx,
+                      int64_t ridx_rs, int kc0, const void* pos, int Qc, int local_w, int S, int kb, int64_t rows,
+                      void* out_vals, int64_t out_vals_rs, int out_off, void* out_idx, int64_t out_idx_rs,
+                      void* final_idx, void* stream);
 int bytes_select_recent(const void* pos, int Qc, int64_t rows, int kb, void* out, void* stream);
 int bytes_select_fill(const void* in, int in_dtype, int64_t in_rs, int k_in, void* out, int out_dtype,
                       int64_t out_rs, int k_out, int64_t rows, const void* pos, int Qc, int64_t S, void* stream);

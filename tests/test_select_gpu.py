@@ -189,3 +189,24 @@ def test_selectors_outside_the_hot_path_raise(dev):
     for sel in ("h2o", "snapkv", "signvq", "sparq", "random"):
         with pytest.raises(ValueError):
             SA.select_topk(sel, q.to(dev), k.to(dev), torch.tensor([63]), 64, 8, 64, 0.1)
+
+
+@pytest.mark.parametrize("S,kb,k_chunk,local_w", [
+    (2100, 513, 1024, 0),        # sort blocks of 512 and 1024; unaligned running list
+    (5000, 1025, 2048, 64),      # eight sorting waves
+    (9000, 2048, 4096, 16),      # the largest sorted selection; rows past 4096 candidates
+    (9000, 2049, 4096, 0),       # one past it: the last step in launches of its own
+    (17000, 300, 16000, 0),      # rows past 8192 candidates
+    (18000, 700, 17000, 9),      # a chunk that no fused step holds
+])
+def test_select_step_sizes(dev, S, kb, k_chunk, local_w):
+    """Fused and separate steps at the edges of their sizes, with heavy ties
+    (scores rounded to few values) and early rows that hold sentinels."""
+    B, Hq, Hk, Qc, D = 1, 3, 1, 3, 64
+    for integer in (False, True):
+        q, k, _ = _inputs(B, Hq, Hk, Qc, S, D, seed=S + kb, integer=integer)
+        pos = torch.tensor([kb // 2, S // 2, S - 1])
+        got = SA.select_topk("exact", q.to(dev), k.to(dev), pos, S, kb, k_chunk, 0.125, local_w=local_w)
+        s = SP.sparse_score_scalar(q.reshape(B, Hq * Qc, 1, D).to(dev), k.to(dev), 0.125).cpu()
+        want = R.select_topk_from_scores(s.reshape(B, Hq, Qc, S), pos, S, kb, k_chunk, local_w)
+        assert torch.equal(got.cpu(), want), integer
