@@ -163,6 +163,32 @@ def lib():
     return _lib
 
 
+class _NoNative:
+    """Stands in where the library has not been built: every call goes on in
+    the Python wrapper, which raises when it comes to launch."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+_native = None
+
+
+def native():
+    """The native call path of the operators (csrc/host/native.cpp): a function
+    returns None where the Python wrapper has to take the call (arguments that
+    need a copy or conversion, errors, a workspace not yet there)."""
+    global _native
+    if _native is None:
+        if not os.path.exists(LIB_PATH):
+            return _NoNative()
+        lib()
+        from . import _native as m
+        m.set_workspaces(_ws)
+        _native = m
+    return _native
+
+
 def check(rc: int, name: str) -> None:
     if rc != 0:
         msg = lib().bytes_error_string(rc)

@@ -11,7 +11,7 @@ from __future__ import annotations
 import torch
 
 from . import _checks as C
-from ._lib import call, ptr, size_query, stream_of, workspace
+from ._lib import call, native, ptr, size_query, stream_of, workspace
 
 
 def decode_attn_bf16(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float = 1.0,
@@ -25,6 +25,9 @@ def decode_attn_bf16(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: f
     1/sqrt(D) for standard attention.  `chunk` forces the split-K chunk
     length in tokens (0 = automatic).
     """
+    out = native().dense(q, k, v, scale, chunk, False)
+    if out is not None:
+        return out
     C.cuda_tensors(q, k, v)
     C.ndim(q, 4, "q"), C.ndim(k, 4, "k"), C.ndim(v, 4, "v")
     for t, n in ((q, "q"), (k, "k"), (v, "v")):
@@ -98,6 +101,9 @@ def decode_attn_fp8(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: fl
     [B,H_k,S,D] float8_e4m3fn, widened to bf16 exactly inside the kernel; fp32
     softmax and accumulation; no scale in the reference (`scale` defaults to
     1.0).  Returns [B,H_q,1,D] in q's dtype (:171)."""
+    out = native().dense(q, k, v, scale, chunk, True)
+    if out is not None:
+        return out
     C.cuda_tensors(q, k, v)
     C.ndim(q, 4, "q"), C.ndim(k, 4, "k"), C.ndim(v, 4, "v")
     C.dtype_in(q, "q", torch.bfloat16)

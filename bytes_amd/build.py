@@ -1,8 +1,9 @@
-"""Build libbytes_amd.so (all HIP kernels + the C ABI) in-tree for gfx950.
+"""Build libbytes_amd.so (all HIP kernels + the C ABI) in-tree for gfx950, and
+_native.so, the operators' native call path over it.
 
-    python -m bytes_amd.build            # compile every csrc/*.hip, link the .so
+    python -m bytes_amd.build            # compile every csrc/*.hip, link the .so files
 
-The library is placed next to this file so that it travels with the source
+The libraries are placed next to this file so that they travel with the source
 tree; nothing is installed anywhere else.
 """
 from __future__ import annotations
@@ -18,6 +19,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libbytes_amd.so")
+NATIVE = os.path.join(HERE, "_native.so")       # the operators' native call path (host code)
 ARCH = "gfx950"
 
 HIPCC = os.environ.get("HIPCC") or shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
@@ -40,6 +42,29 @@ def _compile(src: str) -> str:
     return obj
 
 
+def build_native() -> str:
+    """The extension module csrc/host/native.cpp: host code against torch's
+    headers, linked to libbytes_amd.so beside it."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension as C
+    cxx = os.environ.get("CXX") or shutil.which("g++") or "/opt/rocm/llvm/bin/clang++"
+    tmp = NATIVE + ".tmp"
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           *(f"-isystem{p}" for p in C.include_paths()), "-isystem/opt/rocm/include",
+           f"-isystem{sysconfig.get_paths()['include']}", os.path.join(CSRC, "host", "native.cpp"), "-o", tmp,
+           *(f"-L{p}" for p in C.library_paths()), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip",
+           f"-L{HERE}", "-l:libbytes_amd.so", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"{cxx} failed for csrc/host/native.cpp:\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, NATIVE)
+    return NATIVE
+
+
 def build(verbose: bool = False) -> str:
     os.makedirs(OBJ, exist_ok=True)
     srcs = sorted(glob.glob(os.path.join(CSRC, "*.hip")))
@@ -54,8 +79,9 @@ def build(verbose: bool = False) -> str:
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
     os.replace(tmp, LIB)
+    build_native()
     if verbose:
-        print(f"built {LIB} from {len(srcs)} sources")
+        print(f"built {LIB} from {len(srcs)} sources and {NATIVE}")
     return LIB
 
 

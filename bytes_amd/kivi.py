@@ -13,7 +13,7 @@ import math
 import torch
 
 from . import _checks as C
-from ._lib import call, dtype_code, ptr, size_query, stream_of, workspace
+from ._lib import call, dtype_code, native, ptr, size_query, stream_of, workspace
 
 
 def quantize_and_pack_along_last_dim(data: torch.Tensor, group_size: int, bit: int):
@@ -25,6 +25,9 @@ def quantize_and_pack_along_last_dim(data: torch.Tensor, group_size: int, bit: i
     zero rounded to fp16).  data [..., T] fp16/bf16/fp32 ->
     (code int32 [..., T*bit/32], scale fp16 [..., T/group_size], mn fp16 [..., T/group_size]).
     """
+    out = native().kivi_pack(data, group_size, bit)
+    if out is not None:
+        return out
     C.cuda_tensors(data)
     if bit not in (2, 4):
         raise ValueError(f"bit must be 2 or 4, got {bit}")
@@ -97,6 +100,10 @@ def kivi_decode_attn(Q, Kq, K_scale, K_mn, K_residual, Vq, V_scale, V_mn, V_resi
     (Sq a multiple of 64, at least 1024) on the pipelined kernel with splits
     of -chunk 256-token granules.
     """
+    out = native().kivi(Q, Kq, K_scale, K_mn, K_residual, Vq, V_scale, V_mn, V_residual, bits, group_size, scale,
+                        chunk)
+    if out is not None:
+        return out
     C.cuda_tensors(Q, K_residual, V_residual)
     C.dtype_in(Q, "Q", torch.bfloat16)
     C.dtype_in(K_residual, "K_residual", torch.bfloat16)

@@ -19,7 +19,7 @@ from typing import Optional
 import torch
 
 from . import _checks as C
-from ._lib import call, dtype_code, ptr, size_query, stream_of, workspace
+from ._lib import call, dtype_code, native, ptr, size_query, stream_of, workspace
 
 D_SUB = 8
 
@@ -128,6 +128,9 @@ def decode_attn_pq_kv_fused(q: torch.Tensor, k_centroids: torch.Tensor, k_idx: t
     v_idx [B,H_k,S,M].  Returns [B,H_q,1,D] in v_centroids' dtype."""
     if d_sub_v != D_SUB:
         raise ValueError(f"d_sub_v={d_sub_v} not supported (8)")
+    out = native().pq_fused(q, k_centroids, k_idx, v_idx, v_centroids, scale, chunk)
+    if out is not None:
+        return out
     C.cuda_tensors(q, k_centroids, k_idx, v_idx, v_centroids)
     C.ndim(q, 4, "q"), C.ndim(k_idx, 4, "k_idx")
     C.dtype_in(q, "q", torch.bfloat16)
@@ -272,6 +275,9 @@ def decode_attn_pq_lut_asym(lut: torch.Tensor, k_idx: torch.Tensor, k_out: torch
     k_out [B,H_k,S,C] and q_out [B,H_q,C] (C <= 16; C = 0 allowed); v
     [B,H_k,S,D] bf16 or float8_e4m3fn.  Returns [B,H_q,1,D] in v's dtype, bf16
     for fp8 values (:735)."""
+    out = native().pq_asym(lut, k_idx, k_out, q_out, v, None, None, 0, chunk)
+    if out is not None:
+        return out
     lut, B, Hq, Hk, S, M, K = _lut_checks(lut, k_idx)
     C.cuda_tensors(lut, v)
     k_out, q_out, Cn = _outliers(k_out, q_out, (B, Hk, S), B, Hq)
@@ -331,6 +337,9 @@ def paged_attn_pq_lut_asym(lut: torch.Tensor, k_idx_paged: torch.Tensor, k_out_p
     k_out_paged [num_blocks,H_k,block_size,C], v_paged [num_blocks,H_k,block_size,D]
     bf16 or float8_e4m3fn, q_out [B,H_q,C].  Returns [B,H_q,1,D] in v's dtype,
     bf16 for fp8 values."""
+    out = native().pq_asym(lut, k_idx_paged, k_out_paged, q_out, v_paged, block_table, context_lens, block_size, chunk)
+    if out is not None:
+        return out
     lut, B, Hq, Hk, nblk, bs, M, K = _paged_lut_checks(lut, k_idx_paged)
     if bs != block_size:
         raise ValueError(f"k_idx_paged rows per block {bs} != block_size {block_size}")
@@ -407,6 +416,9 @@ def pq_encode(x: torch.Tensor, centroids: torch.Tensor) -> torch.Tensor:
     the CPU rule of src/quantization.py:203-211 (cdist + argmin).
     x [..., D] (or [H_k, ..., D] with per-head [H_k,M,K,8] centroids).
     Returns uint8 [..., M]."""
+    out = native().pq_encode(x, centroids)
+    if out is not None:
+        return out
     C.cuda_tensors(x, centroids)
     if x.dtype not in (torch.bfloat16, torch.float16, torch.float32):
         raise ValueError(f"x: dtype {x.dtype} not supported")

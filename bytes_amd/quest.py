@@ -14,7 +14,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _checks as C
-from ._lib import call, ptr, size_query, stream_of, workspace
+from ._lib import call, native, ptr, size_query, stream_of, workspace
 from .sparse import _qk_shapes, sparse_gather_attn, topk_indices
 
 
@@ -147,6 +147,9 @@ def quest_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, kb: int, sca
         meta = quest_page_minmax(k, page)
     p = S - 1 if pos is None else int(pos)
     if not return_pages and meta[0].shape[2] <= _SELECT_IN_GATHER_MAX:
+        out = native().quest(q, k, v, kb, scaling, page, meta[0], meta[1], p, local_w)
+        if out is not None:
+            return out
         bound = quest_page_scores(q, meta[0], meta[1], scaling, page=page, pos=p, local_w=local_w)
         return quest_gather_attn(q, k, v, bound, _npick(kb, page, bound.shape[-1]), scaling, page=page,
                                  limit=p + 1)

@@ -11,7 +11,7 @@ from __future__ import annotations
 import torch
 
 from . import _checks as C
-from ._lib import HIP_ERROR_NOT_SUPPORTED, call, lib, ptr, size_query, stream_of, workspace
+from ._lib import call, native, ptr, size_query, stream_of, workspace
 
 TOPK_HIST_ROWS = 1024         # rows whose digit histogram fits the top-k workspace's fixed region
 
@@ -170,6 +170,10 @@ def _topk_workspace(device, rows: int, n: int, k: int) -> torch.Tensor:
 
 
 def _topk(scores: torch.Tensor, k: int, *, sorted: bool, ws=None, hist_ready: bool = False) -> torch.Tensor:
+    if ws is None:
+        out = native().topk(scores, k, bool(sorted))
+        if out is not None:
+            return out
     C.cuda_tensors(scores)
     C.dtype_in(scores, "scores", torch.float32)
     n = scores.shape[-1]
@@ -202,6 +206,9 @@ def sparse_gather_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, idx: t
     clamped to S-1 (the Quest expansion, benchmarks/sparse_attention.py:360-363).
     limit: rows at or past it are masked (the causal bound pos+1; default S).
     """
+    out = native().gather(q, k, v, idx, scaling, chunk, page, limit)
+    if out is not None:
+        return out
     page = int(page)
     if page < 1:
         raise ValueError(f"page={page} must be >= 1")
@@ -251,6 +258,10 @@ def sparse_decode_scalar(q, k_score_or_packed, scale, zero, k_val, v_val, frac, 
     src/attention_kernels.py:1252-1263: bf16 (score_bits=16) or fp8
     (score_bits=8) score keys, or packed 4/2-bit keys with their `scale` and
     `zero` (score_bits=4/2, group_size=32).  Returns [B,H_q,1,D] bf16."""
+    if score_bits in (16, 8) or group_size == 32:
+        out = native().sparse_decode(q, k_score_or_packed, scale, zero, k_val, v_val, frac, scaling, score_bits)
+        if out is not None:
+            return out
     if score_bits in (16, 8):
         scores = sparse_score_scalar(q, k_score_or_packed, scaling, score_bits=score_bits)
     else:
@@ -272,6 +283,9 @@ def token_topk_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, kb: int
     gives them).  Returns (out [B,H_q,1,D] bf16, idx [B,H_k,kb] int32 by
     ascending token index)."""
     ks = k if k_score is None else k_score
+    res = native().token_topk(q, k, v, kb, scaling, ks, score_scale, score_zero, score_bits)
+    if res is not None:
+        return res
     packed = None
     if ks.dtype == torch.uint8:
         if score_bits not in (4, 2) or score_scale is None or score_zero is None:

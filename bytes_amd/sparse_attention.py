@@ -36,7 +36,7 @@ from __future__ import annotations
 import torch
 
 from . import _checks as C
-from ._lib import call, ptr, stream_of
+from ._lib import call, native, ptr, stream_of
 from .quest import quest_page_minmax, quest_page_scores
 from .sparse import _score, _topk, sparse_gather_attn, topk_indices
 
@@ -47,6 +47,18 @@ SCORE_SELECTORS = ("exact", "approx", "int4", "int2", "fp8")
 SELECTORS = SCORE_SELECTORS + ("recent", "quest")
 
 
+def _to_device(host: torch.Tensor, device) -> torch.Tensor:
+    """int64 copy of a host tensor on `device`, through pinned memory and in
+    stream order: a copy from pageable memory holds the host until everything
+    queued on the stream before it has run.  (Under capture the plain copy
+    stays, which refuses: a graph must not read staging memory at replay.)"""
+    if torch.device(device).type != "cuda" or torch.cuda.is_current_stream_capturing():
+        return host.to(device=device, dtype=torch.int64)
+    staged = torch.empty(host.shape, dtype=torch.int64, pin_memory=True)
+    staged.copy_(host)
+    return staged.to(device, non_blocking=True)
+
+
 def _positions(q_pos, Qc: int, device):
     """(int64 positions on `device` [Qc], max position) from an int, a sequence
     or a tensor of Qc positions."""
@@ -55,11 +67,11 @@ def _positions(q_pos, Qc: int, device):
         if p.numel() == 1 and Qc > 1:
             raise ValueError(f"q_pos holds 1 position for Qc={Qc} query rows")
         host = p if p.device.type == "cpu" else None
-        p = p.to(device=device, dtype=torch.int64)
+        p = _to_device(p, device) if host is not None else p.to(device=device, dtype=torch.int64)
     else:
         vals = [int(x) for x in (q_pos if isinstance(q_pos, (list, tuple)) else [q_pos])]
         host = torch.tensor(vals, dtype=torch.int64)
-        p = host.to(device)
+        p = _to_device(host, device)
     if p.numel() != Qc:
         raise ValueError(f"q_pos holds {p.numel()} positions for Qc={Qc} query rows")
     pmax = int((host if host is not None else p).max().item())
@@ -129,8 +141,9 @@ def _stream_select(qf, sel_keys, pos, Qc: int, S: int, kb: int, k_chunk: int, sc
         n = kc1 - kc0
         last = kc1 == max_key
         buf = cand[cur]
-        _score(qf, sel_keys[:, :, kc0:kc1], scaling, group_sum=False,
-               out=buf.view(B, R1, W)[:, :, kbp:kbp + n])
+        keys, dst = sel_keys[:, :, kc0:kc1], buf.view(B, R1, W)[:, :, kbp:kbp + n]
+        if native().score_into(qf, keys, scaling, dst) is None:
+            _score(qf, keys, scaling, group_sum=False, out=dst)
         off = kbp - nrun
         ksel = min(kb, nrun + n)
         nxt = 1 - cur
