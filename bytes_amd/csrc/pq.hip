@@ -33,6 +33,17 @@
 // q . k_hat on MFMA from the staged key codebook rows rather than from LUT
 // entries (within the attention tolerance, not bit-identical to the LUT path).
 //
+// With dense values the general kernel is bound by the instructions of a tile
+// (3.4K cycles for eight waves of 32 tokens, two waves to a SIMD), once two
+// tiles of V rows are in flight and nothing in the loop waits for memory: the
+// block-table entries sit in LDS (read from memory, each was a round trip that
+// the V rows behind it waited for), outlier keys stay raw bits until they are
+// used and only 4 of the 16 possible are loaded where 4 suffice, and a row's
+// offset is computed once and passed between lanes.  8 sequences of 2.7K to 8K
+// tokens, H_q 28, H_k 4, D 128, 4 outlier channels, bf16 values, with the merge:
+// 48.2 us without these, 33 with the table, the channels and two tiles, 30 with
+// the offsets and conflict-free LUT stores, 25 with raw outlier keys.
+//
 // Paged caches (block_table [B, max_blocks] int32, context_lens [B] int32):
 // token t of sequence b is row t % bs of block block_table[b][t / bs]; the
 // block index takes the place of the batch index in every cache stride.  The
@@ -74,6 +85,7 @@ struct PqArgs {
   const int* clens;          // paged: sequence lengths [B]
   int64_t bt_sb;
   int bs, nblk;              // paged: rows per block, blocks in the cache
+  FastDiv dbs;               // division by bs
   int Hk, G, HG, S, K, chunk;   // S: tokens (paged: max_blocks * bs)
   float scale_log2;
   float lut_scale;           // LUTs built in the kernel: entries are lut_scale * (q . codeword)
@@ -85,11 +97,20 @@ __device__ __forceinline__ float load_any(const void* p, int dt, int64_t i) {
                  : (dt == 1 ? (float)static_cast<const _Float16*>(p)[i] : static_cast<const float*>(p)[i]);
 }
 
+// Block-table entries q0 .. of a workgroup's tokens in LDS; n = 0: read the
+// table itself.
+struct PqTable {
+  const int* lds = nullptr;
+  int q0 = 0, n = 0;
+};
+constexpr int kPqTable = 1024;  // entries the general kernel keeps in LDS
+
 // Cache block and row of token t of sequence b.
-__device__ __forceinline__ void pq_locate(const PqArgs& a, int b, int t, int& blk, int& row) {
+__device__ __forceinline__ void pq_locate(const PqArgs& a, int b, int t, int& blk, int& row,
+                                          const PqTable& tab = PqTable()) {
   if (a.btab) {
-    const int q = t / a.bs;
-    blk = min(max(a.btab[(int64_t)b * a.bt_sb + q], 0), a.nblk - 1);
+    const int q = fast_div(t, a.dbs);
+    blk = tab.n ? tab.lds[min(q - tab.q0, tab.n - 1)] : min(max(a.btab[(int64_t)b * a.bt_sb + q], 0), a.nblk - 1);
     row = t - q * a.bs;
   } else {
     blk = b;
@@ -223,7 +244,8 @@ struct PqCfg {
   // per wave: the tile scores, and (dense V) the V tile in the same buffer
   static constexpr int TILE = QV ? SCORES : kTile * D * 2;
   static constexpr int QOUT = QV ? 0 : kPqHeads * kPqOutMax * 4;    // fp32 outlier queries (dense-V modes)
-  static constexpr int kSmem0 = LUT + VCB + kPqWaves * TILE + QOUT;
+  static constexpr int TAB = QV ? 0 : kPqTable * 4;                 // block-table entries (paged)
+  static constexpr int kSmem0 = LUT + VCB + kPqWaves * TILE + QOUT + TAB;
   static constexpr int kEpi = splitk_smem_floats<D, kPqWaves>() * 4;
   static constexpr int kSmem = kSmem0 > kEpi ? kSmem0 : kEpi;
 };
@@ -232,27 +254,30 @@ struct PqCfg {
 //  kc: the M key codes of tile row lane % 32 (every lane scores whole rows)
 //  vc[i]: value code of row p / M, subspace p % M, for staging chunk p = lane + 64*i
 //  vd[i]: dense V chunk p = lane + 64*i (row p / chunks-per-row), bf16 or fp8
-//  ko: the outlier keys of tile row lane % 32
-template <int D, bool QV, bool VF8, bool OUT>
+//  ko: the outlier keys of tile row lane % 32, raw bits (OUT of them: 0, 4 or
+//      kPqOutMax; KO4: 4-byte keys).  They are widened where they are used: a
+//      conversion chosen by dtype right after the load would wait for it, and
+//      with it for every V row in flight
+template <int D, bool QV, bool VF8, int OUT, bool KO4>
 struct PqRegs {
   static constexpr int CPR = VF8 ? D / 16 : D / 8;   // 16-byte V chunks per row
   static constexpr int CPL = kTile * CPR / 64;
   u32x4 kc;
   u32x4 vr[QV ? 2 : 1];   // quantized V: value codes of PV rows hf*16 + lg*4 + (l16 >> 2), hf = 0, 1
   u32x4 vd[QV ? 1 : CPL];
-  float ko[OUT ? kPqOutMax : 1];
+  uint32_t ko[OUT ? OUT : 1];
 };
 
 // Issue the tile at t0 (rows clamped to len - 1).  Each lane locates its own
 // row lane % 32; rows of the V chunks come from the owning lane by shuffle.
-template <int D, bool QV, bool VF8, bool OUT>
+template <int D, bool QV, bool VF8, int OUT, bool KO4>
 __device__ __forceinline__ void pq_issue(const PqArgs& a, int b, const uint8_t* kih, const uint8_t* vih,
                                          const char* vh, const char* koh, int len, int t0, int lane,
-                                         PqRegs<D, QV, VF8, OUT>& r) {
-  using R = PqRegs<D, QV, VF8, OUT>;
+                                         const PqTable& tab, PqRegs<D, QV, VF8, OUT, KO4>& r) {
+  using R = PqRegs<D, QV, VF8, OUT, KO4>;
   constexpr int M = D / 8;
   int blk, row;
-  pq_locate(a, b, min(t0 + (lane & 31), len - 1), blk, row);
+  pq_locate(a, b, min(t0 + (lane & 31), len - 1), blk, row, tab);
   {
     const uint8_t* p = kih + (int64_t)blk * a.ki_sb + (int64_t)row * a.ki_ss;
     if constexpr (M == 16) {
@@ -262,19 +287,29 @@ __device__ __forceinline__ void pq_issue(const PqArgs& a, int b, const uint8_t* 
       r.kc = u32x4{h[0], h[1], 0u, 0u};
     }
   }
-  if constexpr (OUT) {
+  if constexpr (OUT > 0) {
     // channels past C read channel C - 1; their query weights are zero
     const int64_t o = (int64_t)blk * a.ko_sb + (int64_t)row * a.ko_ss;
 #pragma unroll
-    for (int c = 0; c < kPqOutMax; ++c) r.ko[c] = load_any(koh, a.ko_dt, o + min(c, a.C - 1));
+    for (int c = 0; c < OUT; ++c) {
+      const int64_t e = o + min(c, a.C - 1);
+      if constexpr (KO4) r.ko[c] = reinterpret_cast<const uint32_t*>(koh)[e];
+      else r.ko[c] = reinterpret_cast<const uint16_t*>(koh)[e];
+    }
   }
+  // a value row's offset is computed by the lane that located the row and
+  // passed to the lanes that read it
+  auto from = [](int64_t o, int rr) {
+    const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)o, rr, 64), hi = (uint32_t)__shfl((int)(uint32_t)((uint64_t)o >> 32), rr, 64);
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+  };
   if constexpr (QV) {
     const int l16 = lane & 15, lg = lane >> 4;
+    const int64_t vo = (int64_t)blk * a.vi_sb + (int64_t)row * a.vi_ss;
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf) {
       const int rr = hf * 16 + lg * 4 + (l16 >> 2);
-      const int bq = __shfl(blk, rr, 64), rq = __shfl(row, rr, 64);
-      const uint8_t* p = vih + (int64_t)bq * a.vi_sb + (int64_t)rq * a.vi_ss;
+      const uint8_t* p = vih + from(vo, rr);
       if constexpr (M == 16) {
         r.vr[hf] = ld16(p);
       } else {
@@ -284,12 +319,12 @@ __device__ __forceinline__ void pq_issue(const PqArgs& a, int b, const uint8_t* 
     }
   } else {
     constexpr int ES = VF8 ? 1 : 2;
+    const int64_t vo = ((int64_t)blk * a.v_sb + (int64_t)row * a.v_ss) * ES;
 #pragma unroll
     for (int i = 0; i < R::CPL; ++i) {
       const int p = lane + 64 * i;
       const int rr = p / R::CPR, pos = p - rr * R::CPR;
-      const int bq = __shfl(blk, rr, 64), rq = __shfl(row, rr, 64);
-      r.vd[i] = ld16(vh + ((int64_t)bq * a.v_sb + (int64_t)rq * a.v_ss) * ES + pos * 16);
+      r.vd[i] = ld16(vh + from(vo, rr) + pos * 16);
     }
   }
 }
@@ -308,9 +343,9 @@ struct CodebookV {
   }
 };
 
-template <int D, bool QV, bool VF8, bool OUT>
-__device__ __forceinline__ void pq_stage_dense_v(int lane, const PqRegs<D, QV, VF8, OUT>& r, char* vst) {
-  using R = PqRegs<D, QV, VF8, OUT>;
+template <int D, bool QV, bool VF8, int OUT, bool KO4>
+__device__ __forceinline__ void pq_stage_dense_v(int lane, const PqRegs<D, QV, VF8, OUT, KO4>& r, char* vst) {
+  using R = PqRegs<D, QV, VF8, OUT, KO4>;
 #pragma unroll
   for (int i = 0; i < R::CPL; ++i) {
     const int p = lane + 64 * i;
@@ -333,8 +368,8 @@ __device__ __forceinline__ void pq_stage_dense_v(int lane, const PqRegs<D, QV, V
 // score-MFMA layout (head l%16, rows blk*16 + lg*4 + i) and the softmax/PV
 // step runs: quantized V straight from the codebook in LDS, dense V staged in
 // the same buffer first.
-template <int D, bool QV, bool VF8, bool OUT>
-__device__ __forceinline__ void pq_tile(const PqArgs& a, const PqRegs<D, QV, VF8, OUT>& r, uint32_t vmask, int lane,
+template <int D, bool QV, bool VF8, int OUT, bool KO4>
+__device__ __forceinline__ void pq_tile(const PqArgs& a, const PqRegs<D, QV, VF8, OUT, KO4>& r, uint32_t vmask, int lane,
                                         int nh, const float* lut, const char* vcb, const float* qo, char* vst,
                                         float& m_run, float& l_run, f32x4 (&acc)[D / 16]) {
   constexpr int M = D / 8;
@@ -352,15 +387,24 @@ __device__ __forceinline__ void pq_tile(const PqArgs& a, const PqRegs<D, QV, VF8
     const uint32_t code = (w >> ((jj & 3) * 8)) & 0xFFu;
     ps += *reinterpret_cast<const f32x4*>(lut + ((hf * MH + jj) * kPqKMax + code) * kPqHeads);
   }
+  float ko[OUT ? OUT : 1];
+  if constexpr (OUT > 0) {
+    const bool bf = a.ko_dt == 0;
+#pragma unroll
+    for (int c = 0; c < OUT; ++c) {
+      if constexpr (KO4) ko[c] = __uint_as_float(r.ko[c]);
+      else ko[c] = bf ? bf16_bits_to_f32((uint16_t)r.ko[c]) : (float)__builtin_bit_cast(_Float16, (uint16_t)r.ko[c]);
+    }
+  }
   f32x4 sc4;
 #pragma unroll
   for (int h = 0; h < kPqHeads; ++h) {
     const float o = shfl_xor_f(ps[h], 32);
     sc4[h] = hf ? o + ps[h] : ps[h] + o;
-    if constexpr (OUT) {
+    if constexpr (OUT > 0) {
       float so = 0.f;
 #pragma unroll
-      for (int c = 0; c < kPqOutMax; ++c) so += qo[h * kPqOutMax + c] * r.ko[c];   // zero past C
+      for (int c = 0; c < OUT; ++c) so += qo[h * kPqOutMax + c] * ko[c];   // zero past C
       sc4[h] += so;
     }
   }
@@ -383,7 +427,7 @@ __device__ __forceinline__ void pq_tile(const PqArgs& a, const PqRegs<D, QV, VF8
   } else {
     // V tile into the same buffer
     wave_lds_sync();
-    pq_stage_dense_v<D>(lane, r, vst);
+    pq_stage_dense_v<D, QV, VF8, OUT, KO4>(lane, r, vst);
     wave_lds_sync();
     tile_softmax_pv<D, false>(s, l16 < nh ? vmask : 0u, a.scale_log2, lane, vst, m_run, l_run, acc);
   }
@@ -404,10 +448,10 @@ __device__ __forceinline__ void stage_chunks(int n, SRC src, DST dst) {
   }
 }
 
-template <int D, bool BUILD_LUT, bool QV, bool VF8, bool OUT>
+template <int D, bool BUILD_LUT, bool QV, bool VF8, int OUT, bool KO4>
 __global__ __launch_bounds__(kPqWaves * 64, 1) void pq_decode_kernel(PqArgs a) {
   using C = PqCfg<D, QV>;
-  using Regs = PqRegs<D, QV, VF8, OUT>;
+  using Regs = PqRegs<D, QV, VF8, OUT, KO4>;
   constexpr int M = D / 8;
   __shared__ __attribute__((aligned(16))) char smem_raw[C::kSmem];
   float* lut = reinterpret_cast<float*>(smem_raw);
@@ -437,8 +481,21 @@ __global__ __launch_bounds__(kPqWaves * 64, 1) void pq_decode_kernel(PqArgs a) {
   // len - 1 past the end), so each wait counts the same requests.
   LutQ<D> qrow;
   if (BUILD_LUT && w < kPqHeads) qrow = lut_load_q<D>(a.q + (int64_t)b * a.q_sb + (int64_t)hq0 * a.q_sh, a.q_sh, w, nh);
+  // Paged, dense values: the table entries of this workgroup's tokens are
+  // staged in LDS (the tile loop then finds its rows without a memory round
+  // trip, whose wait would also be one for every V row in flight).
+  PqTable tab;
+  int* tab_lds = reinterpret_cast<int*>(smem_raw + C::LUT + C::VCB + kPqWaves * C::TILE + C::QOUT);
+  int tab_n = 0, tab_q0 = 0;
+  if (!QV && a.btab && t_begin < t_end) {
+    tab_q0 = fast_div(t_begin, a.dbs);
+    tab_n = fast_div(t_end - 1, a.dbs) - tab_q0 + 1;
+    if (tab_n > kPqTable) tab_n = 0;
+    for (int e = threadIdx.x; e < tab_n; e += kPqWaves * 64)
+      tab_lds[e] = min(max(a.btab[(int64_t)b * a.bt_sb + tab_q0 + e], 0), a.nblk - 1);
+  }
   Regs r;
-  if (any) pq_issue<D, QV, VF8, OUT>(a, b, kih, vih, vh, koh, len, t, lane, r);
+  if (any) pq_issue<D, QV, VF8, OUT, KO4>(a, b, kih, vih, vh, koh, len, t, lane, tab, r);
 
   // The value codebook (quantized V) is requested now, with the first tile's
   // codes, so it arrives while the LUTs are built or staged; it is stored to
@@ -490,26 +547,30 @@ __global__ __launch_bounds__(kPqWaves * 64, 1) void pq_decode_kernel(PqArgs a) {
     }
   } else {
     // the caller's LUTs, transposed so the heads of one (subspace, code) are
-    // adjacent; chunks past n repeat the last one (same values, same place)
-    const int K4 = K / 4, n = nh * M * K4;
-    constexpr int NT = kPqWaves * 64, BATCH = 8;
-    for (int e0 = threadIdx.x; e0 < n; e0 += NT * BATCH) {
-      u32x4 v[BATCH];
+    // adjacent: a thread reads one entry of each head (consecutive lanes,
+    // consecutive codes) and stores the four together (16 bytes, no bank
+    // conflicts; four-code chunks of one head scattered as single words put 16
+    // lanes on a bank).  Entries past M * K repeat the last one, heads past nh
+    // repeat head nh - 1: nothing sits under a lane mask, and heads past nh
+    // are never read.
+    const int n = M * K;
+    constexpr int NT = kPqWaves * 64, BATCH = M * kPqKMax / NT;
+    const float* lb = a.lut + (int64_t)b * a.l_sb + (int64_t)hq0 * a.l_sh;
+    const float* lh[kPqHeads];
 #pragma unroll
-      for (int bb = 0; bb < BATCH; ++bb) {
-        const int e = min(e0 + bb * NT, n - 1);
-        const int h = e / (M * K4), r2 = e - h * (M * K4);
-        const int j = r2 / K4, c4 = r2 - j * K4;
-        v[bb] = ld16(a.lut + (int64_t)b * a.l_sb + (int64_t)(hq0 + h) * a.l_sh + j * K + c4 * 4);
-      }
+    for (int h = 0; h < kPqHeads; ++h) lh[h] = lb + (int64_t)min(h, nh - 1) * a.l_sh;
+    f32x4 v[BATCH];
 #pragma unroll
-      for (int bb = 0; bb < BATCH; ++bb) {
-        const int e = min(e0 + bb * NT, n - 1);
-        const int h = e / (M * K4), r2 = e - h * (M * K4);
-        const int j = r2 / K4, c4 = r2 - j * K4;
+    for (int bb = 0; bb < BATCH; ++bb) {
+      const int e = min((int)threadIdx.x + bb * NT, n - 1);
 #pragma unroll
-        for (int x = 0; x < 4; ++x) lut[(j * kPqKMax + c4 * 4 + x) * kPqHeads + h] = __uint_as_float(v[bb][x]);
-      }
+      for (int h = 0; h < kPqHeads; ++h) v[bb][h] = lh[h][e];
+    }
+#pragma unroll
+    for (int bb = 0; bb < BATCH; ++bb) {
+      const int e = min((int)threadIdx.x + bb * NT, n - 1);
+      const int j = e / K, c = e - j * K;
+      *reinterpret_cast<f32x4*>(lut + (j * kPqKMax + c) * kPqHeads) = v[bb];
     }
   }
   if constexpr (QV) {
@@ -521,7 +582,7 @@ __global__ __launch_bounds__(kPqWaves * 64, 1) void pq_decode_kernel(PqArgs a) {
     }
   }
   float* qo = reinterpret_cast<float*>(smem_raw + C::LUT + C::VCB + kPqWaves * C::TILE);
-  if constexpr (OUT) {
+  if constexpr (OUT > 0) {
     for (int e = threadIdx.x; e < kPqHeads * kPqOutMax; e += kPqWaves * 64) {
       const int h = e / kPqOutMax, c = e - h * kPqOutMax;
       qo[e] = (h < nh && c < a.C) ? load_any(a.qout, a.qo_dt, (int64_t)b * a.qo_sb + (int64_t)(hq0 + h) * a.qo_sh + c)
@@ -536,13 +597,32 @@ __global__ __launch_bounds__(kPqWaves * 64, 1) void pq_decode_kernel(PqArgs a) {
 
   __syncthreads();
   if (any) {
-    // tile t runs on the registers that arrived during the last tile, which
-    // are copied out first and refilled with tile t+STEP (clamped past the end)
-    for (; t < t_end; t += STEP) {
-      const Regs cur = r;
-      pq_issue<D, QV, VF8, OUT>(a, b, kih, vih, vh, koh, len, t + STEP, lane, r);
-      wave_lds_sync();
-      pq_tile<D, QV, VF8, OUT>(a, cur, range_mask(t, t_end), lane, nh, lut, vcb, qo, vst, m_run, l_run, acc);
+    // tile t runs on the registers that arrived during the last tiles, which
+    // are copied out first and refilled with a tile further on (clamped past
+    // the end): the next one, or with dense values the one after it, so two
+    // tiles of V rows are in flight per wave
+    if constexpr (QV) {
+      for (; t < t_end; t += STEP) {
+        const Regs cur = r;
+        pq_issue<D, QV, VF8, OUT, KO4>(a, b, kih, vih, vh, koh, len, t + STEP, lane, tab, r);
+        wave_lds_sync();
+        pq_tile<D, QV, VF8, OUT, KO4>(a, cur, range_mask(t, t_end), lane, nh, lut, vcb, qo, vst, m_run, l_run, acc);
+      }
+    } else {
+      // (rows clamped to t_end - 1, the last token of the staged entries)
+      tab = PqTable{tab_lds, tab_q0, tab_n};
+      Regs r1;
+      pq_issue<D, QV, VF8, OUT, KO4>(a, b, kih, vih, vh, koh, t_end, t + STEP, lane, tab, r1);
+      auto step = [&](Regs& x) {
+        const Regs cur = x;
+        pq_issue<D, QV, VF8, OUT, KO4>(a, b, kih, vih, vh, koh, t_end, t + 2 * STEP, lane, tab, x);
+        wave_lds_sync();
+        pq_tile<D, QV, VF8, OUT, KO4>(a, cur, range_mask(t, t_end), lane, nh, lut, vcb, qo, vst, m_run, l_run, acc);
+        t += STEP;
+        return t < t_end;
+      };
+      while (step(r) && step(r1)) {
+      }
     }
   }
   splitk_epilogue<D, kPqWaves>(m_run, l_run, acc, reinterpret_cast<float*>(smem_raw), a.o, unit, split, b, hq0, nh,
@@ -1427,22 +1507,28 @@ static int pq_launch(PqArgs& a, int mode, bool vf8, int B, int Hq, int Hk, int S
   a.o.Hk = Hk; a.o.HB = a.HG; a.o.G = a.G; a.o.hbs = kPqHeads;
   splitk_carve(workspace, units, ns, a.o);
   dim3 grid((unsigned)(ns * units)), block(kPqWaves * 64);
-  const bool outl = a.C > 0;
-#define PQ_LAUNCH(DD, BL, QQ, F8, OU) BYTES_LAUNCH(kProfPq, (pq_decode_kernel<DD, BL, QQ, F8, OU>), grid, block, 0, st, a)
-#define PQ_MODES(DD)                                          \
-  if (mode == 0) PQ_LAUNCH(DD, false, true, false, false);    \
-  else if (mode == 2) PQ_LAUNCH(DD, true, false, false, false); \
-  else if (mode == 3) PQ_LAUNCH(DD, true, true, false, false); \
-  else if (!vf8 && !outl) PQ_LAUNCH(DD, false, false, false, false); \
-  else if (!vf8) PQ_LAUNCH(DD, false, false, false, true);   \
-  else if (!outl) PQ_LAUNCH(DD, false, false, true, false);  \
-  else PQ_LAUNCH(DD, false, false, true, true);
+  // outlier channels a tile keeps per row: none, up to 4, up to kPqOutMax
+#define PQ_LAUNCH(DD, BL, QQ, F8, OU, K4) \
+  BYTES_LAUNCH(kProfPq, (pq_decode_kernel<DD, BL, QQ, F8, OU, K4>), grid, block, 0, st, a)
+#define PQ_OUT(DD, F8)                                                      \
+  if (a.C == 0) PQ_LAUNCH(DD, false, false, F8, 0, false);                  \
+  else if (a.C <= 4 && a.ko_dt != 2) PQ_LAUNCH(DD, false, false, F8, 4, false); \
+  else if (a.C <= 4) PQ_LAUNCH(DD, false, false, F8, 4, true);              \
+  else if (a.ko_dt != 2) PQ_LAUNCH(DD, false, false, F8, kPqOutMax, false); \
+  else PQ_LAUNCH(DD, false, false, F8, kPqOutMax, true);
+#define PQ_MODES(DD)                                                  \
+  if (mode == 0) PQ_LAUNCH(DD, false, true, false, 0, false);         \
+  else if (mode == 2) PQ_LAUNCH(DD, true, false, false, 0, false);    \
+  else if (mode == 3) PQ_LAUNCH(DD, true, true, false, 0, false);     \
+  else if (!vf8) { PQ_OUT(DD, false) }                                \
+  else { PQ_OUT(DD, true) }
   if (D == 128) {
     PQ_MODES(128)
   } else {
     PQ_MODES(64)
   }
 #undef PQ_MODES
+#undef PQ_OUT
 #undef PQ_LAUNCH
   int rc = (int)hipGetLastError();
   if (rc) return rc;
@@ -1540,6 +1626,7 @@ int bytes_pq_lut_decode_attn(const void* lut, int64_t l_sb, int64_t l_sh, const 
   a.bt_sb = bt_sb;
   a.clens = context_lens;
   a.bs = block_size;
+  a.dbs = make_fastdiv((uint32_t)(block_size > 0 ? block_size : 1));
   a.nblk = num_blocks;
   return pq_launch(a, qv ? 0 : 1, v_fp8 != 0, B, Hq, Hk, S, D, K, out, out_dtype, o_sb, o_sh, scale, chunk_req,
                    workspace, workspace_bytes, stream);

@@ -155,3 +155,27 @@ def test_asym_argument_errors(dev):
                                    torch.zeros(1, 4, 17, device=dev), args[4])          # 17 outlier channels
     with pytest.raises(ValueError):
         PQ.decode_attn_pq_lut_asym(args[0], args[1], args[2], args[3][:, :2], args[4])  # q_out heads
+
+
+@pytest.mark.parametrize("bs,C,ko_dtype,v_dtype,lens", [
+    (1, 2, torch.bfloat16, torch.bfloat16, [1500, 7]),      # more table entries than the kernel keeps in LDS
+    (16, 4, torch.float16, F8, [513, 512, 1]),              # a tile past a tile-pair's end
+    (24, 5, torch.bfloat16, torch.bfloat16, [700, 255]),    # blocks that split tiles; the 16-channel kernel
+    (16, 3, torch.float32, F8, [257, 1025]),                # 4-byte outliers, few channels
+    (32, 16, torch.float32, torch.bfloat16, [300]),
+])
+def test_paged_asym_tables_and_channels(dev, bs, C, ko_dtype, v_dtype, lens):
+    """Block tables in LDS and past its size, every outlier width, an odd and
+    an even number of tiles per wave, against the oracle; one split of all
+    tokens against the automatic plan."""
+    B, Hq, Hk, D = len(lens), 14, 2, 128
+    S = max(lens)
+    lut, k_idx, k_out, q_out, v = _asym_inputs(B, Hq, Hk, S, D, C, 64, seed=S + C, v_dtype=v_dtype)
+    k_out = k_out.to(ko_dtype)
+    (kp, kop, vp), table = _paginate([k_idx, k_out, v], lens, bs, seed=bs)
+    cl = torch.tensor(lens, dtype=torch.int32)
+    ref = R.paged_attn_pq_lut_asym(lut, kp, kop, q_out, vp, table, cl, bs)
+    for chunk in (0, 2048):
+        out = PQ.paged_attn_pq_lut_asym(lut.to(dev), kp.to(dev), kop.to(dev), q_out.to(dev), vp.to(dev),
+                                        table.to(dev), cl.to(dev), block_size=bs, chunk=chunk)
+        _check(out, ref, f"bs {bs} C {C} {ko_dtype} {v_dtype} chunk {chunk}")
