@@ -73,6 +73,12 @@ SIGNATURES: Dict[str, Tuple] = {
         c_i64, c_i64,                                 # idx strides (b, h)
         c_i64, c_i64,                                 # out strides
         c_f32, c_int, c_vp, c_sz, c_vp),              # scaling, chunk, workspace, bytes, stream
+    "bytes_attend_topk": (
+        c_vp, c_vp, c_vp, c_int, c_vp, c_vp, c_int, c_vp,       # q, k, v, k/v are fp8, idx, pos, Qc, out
+        c_int, c_int, c_int, c_int, c_int, c_int,               # B, Hq, Hk, S, D, kb
+        c_i64, c_i64, c_i64, c_i64, c_i64, c_i64, c_i64, c_i64,   # q (b, h), k (b, h, s), v (b, h, s) strides
+        c_i64, c_i64, c_i64, c_i64,                             # idx, out strides (b, h)
+        c_f32, c_vp, c_sz, c_vp),                               # scaling, workspace, bytes, stream
     "bytes_quest_gather_attn": (
         c_vp, c_vp, c_vp, c_int, c_vp, c_i64, c_i64,  # q, k, v, k/v are fp8, bound, bound strides (b, h)
         c_int, c_int, c_vp,                           # np, npick, out

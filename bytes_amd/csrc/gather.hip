@@ -43,6 +43,10 @@ struct GatherArgs {
   int Hk, G, HB, S, kb, chunk, per_head;
   int page;                  // 0: idx holds rows; > 0: idx holds page ids of `page` rows each
   int limit;                 // rows >= limit take no part
+  const int64_t* idx64;      // per-head lists of int64 entries instead (strides i_sb, i_sh), entries past
+  const int64_t* pos;        // the head's query position pos[head % Qc] taking no part
+  int Qc;
+  bool nt;                   // K/V rows with the non-temporal hint
   const float* bound;        // Quest selection: page bounds [B, Hq, np] (row strides b_sb, b_sh)
   int64_t b_sb, b_sh;
   int np;
@@ -67,8 +71,15 @@ struct GatherCfg {
 };
 
 // Loads of one 32-row tile whose rows are rows[j0 .. j0+31] (entries past n or
-// negative read row 0: same instructions every tile, no divergence).
-template <int D>
+// negative read row 0: same instructions every tile, no divergence).  NT: with
+// the non-temporal hint, for rows read once; without it for rows that other
+// lists name too and that stay in L2.
+template <bool NT>
+__device__ __forceinline__ u32x4 gather_ld16(const void* p) {
+  return NT ? ld16_nt(p) : ld16(p);
+}
+
+template <int D, bool NT>
 __device__ __forceinline__ void gather_issue(const uint16_t* kbase, const uint16_t* vbase, int64_t k_ss,
                                              int64_t v_ss, const int32_t* rows, int j0, int n, int lane,
                                              DenseRegs<D>& r) {
@@ -80,12 +91,12 @@ __device__ __forceinline__ void gather_issue(const uint16_t* kbase, const uint16
     const int j = j0 + rr;
     int row = j < n ? rows[j] : 0;
     row = row < 0 ? 0 : row;
-    r.k[i] = ld16_nt(kbase + (int64_t)row * k_ss + pos * 8);
-    r.v[i] = ld16_nt(vbase + (int64_t)row * v_ss + pos * 8);
+    r.k[i] = gather_ld16<NT>(kbase + (int64_t)row * k_ss + pos * 8);
+    r.v[i] = gather_ld16<NT>(vbase + (int64_t)row * v_ss + pos * 8);
   }
 }
 
-template <int D>
+template <int D, bool NT>
 __device__ __forceinline__ void gather_issue_fp8(const uint8_t* kbase, const uint8_t* vbase, int64_t k_ss,
                                                  int64_t v_ss, const int32_t* rows, int j0, int n, int lane,
                                                  DenseRegs8<D>& r) {
@@ -97,13 +108,13 @@ __device__ __forceinline__ void gather_issue_fp8(const uint8_t* kbase, const uin
     const int j = j0 + rr;
     int row = j < n ? rows[j] : 0;
     row = row < 0 ? 0 : row;
-    r.k[i] = ld16_nt(kbase + (int64_t)row * k_ss + pos * 16);
-    r.v[i] = ld16_nt(vbase + (int64_t)row * v_ss + pos * 16);
+    r.k[i] = gather_ld16<NT>(kbase + (int64_t)row * k_ss + pos * 16);
+    r.v[i] = gather_ld16<NT>(vbase + (int64_t)row * v_ss + pos * 16);
   }
 }
 
 // SEL > 0: Quest selection in the prologue, SEL bounds per thread.
-template <int D, bool FP8, int SEL>
+template <int D, bool FP8, int SEL, bool NT>
 __global__ __launch_bounds__(kGatherWaves * 64, 2) void gather_decode_kernel(GatherArgs a) {
   using C = DenseCfg<D>;
   __shared__ __attribute__((aligned(16))) char smem_raw[GatherCfg<D>::kSmem];
@@ -139,7 +150,7 @@ __global__ __launch_bounds__(kGatherWaves * 64, 2) void gather_decode_kernel(Gat
   // (block_select) and lists them, ascending, in LDS
   int32_t* pids = reinterpret_cast<int32_t*>(smem_raw + GatherCfg<D>::kSelWs * 4);
   if constexpr (SEL > 0) {
-    constexpr int NT = kGatherWaves * 64;
+    constexpr int kNT = kGatherWaves * 64;
     const float* bsrc = a.bound + (int64_t)b * a.b_sb + (int64_t)hq0 * a.b_sh;
     uint32_t key[SEL];
     // all of a thread's loads in flight together (indices clamped to the
@@ -161,13 +172,21 @@ __global__ __launch_bounds__(kGatherWaves * 64, 2) void gather_decode_kernel(Gat
       for (int u = 0; u < SEL; ++u) key[u] = score_order_key(bv[u]);
     }
     uint32_t* ws = reinterpret_cast<uint32_t*>(smem_raw);
-    const BlockSel sel = block_select<NT, SEL>(key, a.np, a.kb / a.page, ws);
-    block_select_emit<NT, SEL>(key, a.np, sel, ws, [&](uint32_t pos, int idx, uint32_t) { pids[pos] = idx; });
+    const BlockSel sel = block_select<kNT, SEL>(key, a.np, a.kb / a.page, ws);
+    block_select_emit<kNT, SEL>(key, a.np, sel, ws, [&](uint32_t pos, int idx, uint32_t) { pids[pos] = idx; });
     __syncthreads();
   }
 
   const int p_begin = split * a.chunk;
   const int n = min(a.chunk, a.kb - p_begin);
+  if (SEL == 0 && a.idx64) {
+    const int64_t p = a.pos[hq0 % a.Qc], lim = p < a.limit - 1 ? p : a.limit - 1;
+    const int64_t* i64 = a.idx64 + (int64_t)b * a.i_sb + (int64_t)hq0 * a.i_sh + p_begin;
+    for (int i = threadIdx.x; i < n; i += kGatherWaves * 64) {
+      const int64_t r = i64[i];
+      rows[i] = r >= 0 && r <= lim ? (int)r : -1;
+    }
+  } else
   for (int i = threadIdx.x; i < n; i += kGatherWaves * 64) {
     const int j = p_begin + i;
     int64_t r;
@@ -201,8 +220,8 @@ __global__ __launch_bounds__(kGatherWaves * 64, 2) void gather_decode_kernel(Gat
     const Elem* vbase = static_cast<const Elem*>(a.v) + (int64_t)b * a.v_sb + (int64_t)hk * a.v_sh;
     Regs r;
     auto issue = [&](int j0) {
-      if constexpr (FP8) gather_issue_fp8<D>(kbase, vbase, a.k_ss, a.v_ss, rows, j0, n, lane, r);
-      else gather_issue<D>(kbase, vbase, a.k_ss, a.v_ss, rows, j0, n, lane, r);
+      if constexpr (FP8) gather_issue_fp8<D, NT>(kbase, vbase, a.k_ss, a.v_ss, rows, j0, n, lane, r);
+      else gather_issue<D, NT>(kbase, vbase, a.k_ss, a.v_ss, rows, j0, n, lane, r);
     };
     issue(j);
     for (; j < n; j += STEP) {
@@ -240,9 +259,10 @@ static void gather_plan(int kb, long units, int chunk_req, int* chunk, int* ns) 
 }
 
 static void gather_launch(const GatherArgs& a, int D, int kv_fp8, dim3 grid, dim3 block, hipStream_t st) {
-#define GL(DD, F8, SL) BYTES_LAUNCH(kProfGather, (gather_decode_kernel<DD, F8, SL>), grid, block, 0, st, a)
+#define GL(DD, F8, SL) BYTES_LAUNCH(kProfGather, (gather_decode_kernel<DD, F8, SL, true>), grid, block, 0, st, a)
 #define GL_SEL(DD, F8)                  \
-  if (!a.bound) GL(DD, F8, 0);          \
+  if (!a.bound && !a.nt) BYTES_LAUNCH(kProfGather, (gather_decode_kernel<DD, F8, 0, false>), grid, block, 0, st, a); \
+  else if (!a.bound) GL(DD, F8, 0);     \
   else if (a.np <= 1024) GL(DD, F8, 4); \
   else if (a.np <= 2048) GL(DD, F8, 8); \
   else GL(DD, F8, 16);
@@ -264,25 +284,13 @@ static long gather_units(int B, int Hq, int Hk, int per_head) {
 
 using namespace bytes_amd;
 
-extern "C" {
-
-int bytes_gather_attn_workspace_size(int B, int Hq, int Hk, int kb, int D, int per_head, int chunk_req,
-                                     size_t* bytes) {
-  if (!bytes || B <= 0 || Hk <= 0 || Hq <= 0 || Hq % Hk != 0 || kb <= 0) return (int)hipErrorInvalidValue;
-  if (D != 64 && D != 128) return (int)hipErrorInvalidValue;
-  const long units = gather_units(B, Hq, Hk, per_head);
-  int chunk, ns;
-  gather_plan(kb, units, chunk_req, &chunk, &ns);
-  *bytes = splitk_workspace_bytes(units, ns, D);
-  return 0;
-}
-
-int bytes_gather_attn(const void* q, const void* k, const void* v, int kv_fp8, const void* idx, void* out, int B,
-                      int Hq, int Hk, int S, int D, int kb, int per_head, int page, int limit, int64_t q_sb, int64_t q_sh,
-                      int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss, int64_t i_sb, int64_t i_sh,
-                      int64_t o_sb, int64_t o_sh, float scaling, int chunk_req, void* workspace,
-                      size_t workspace_bytes, void* stream) {
-  if (!q || !k || !v || !idx || !out || B <= 0 || Hk <= 0 || Hq <= 0 || Hq % Hk != 0 || S <= 0 || kb <= 0)
+static int gather_attn(const void* q, const void* k, const void* v, int kv_fp8, const void* idx, const void* idx64,
+                       const void* pos, int Qc, void* out, int B, int Hq, int Hk, int S, int D, int kb, int per_head,
+                       int page, int limit, int64_t q_sb, int64_t q_sh, int64_t k_sb, int64_t k_sh, int64_t k_ss,
+                       int64_t v_sb, int64_t v_sh, int64_t v_ss, int64_t i_sb, int64_t i_sh, int64_t o_sb,
+                       int64_t o_sh, float scaling, int chunk_req, void* workspace, size_t workspace_bytes,
+                       void* stream) {
+  if (!q || !k || !v || (!idx && !idx64) || !out || B <= 0 || Hk <= 0 || Hq <= 0 || Hq % Hk != 0 || S <= 0 || kb <= 0)
     return (int)hipErrorInvalidValue;
   if (D != 64 && D != 128) return (int)hipErrorInvalidValue;
   if (page < 0 || (page > 0 && kb % page != 0) || limit < 0 || limit > S) return (int)hipErrorInvalidValue;
@@ -302,6 +310,16 @@ int bytes_gather_attn(const void* q, const void* k, const void* v, int kv_fp8, c
   a.v = v;
   a.v_sb = v_sb; a.v_sh = v_sh; a.v_ss = v_ss;
   a.idx = static_cast<const int32_t*>(idx);
+  a.idx64 = static_cast<const int64_t*>(idx64);
+  a.pos = static_cast<const int64_t*>(pos);
+  a.Qc = Qc;
+  // Rows are read again and again where the lists of a KV head's query heads
+  // hold several times its cache and the cache fits an XCD's 4 MB of L2 beside
+  // its neighbours': 3584 lists of 819 rows over two 1 MB caches take 58 us
+  // with plain loads and 69 with the hint, 2048 lists over 256 caches of 8 MB
+  // 132 and 127.
+  const int64_t cache = (int64_t)S * D * (kv_fp8 ? 2 : 4);
+  a.nt = !(per_head && (int64_t)(Hq / Hk) * kb >= 4 * (int64_t)S && cache <= (4 << 20));
   a.i_sb = i_sb; a.i_sh = i_sh;
   a.Hk = Hk; a.G = Hq / Hk; a.HB = (a.G + 15) / 16; a.S = S; a.kb = kb;
   a.per_head = per_head ? 1 : 0;
@@ -327,6 +345,40 @@ int bytes_gather_attn(const void* q, const void* k, const void* v, int kv_fp8, c
   int rc = (int)hipGetLastError();
   if (rc) return rc;
   return splitk_combine(a.o, units, D, st);
+}
+
+
+extern "C" {
+
+int bytes_gather_attn_workspace_size(int B, int Hq, int Hk, int kb, int D, int per_head, int chunk_req,
+                                     size_t* bytes) {
+  if (!bytes || B <= 0 || Hk <= 0 || Hq <= 0 || Hq % Hk != 0 || kb <= 0) return (int)hipErrorInvalidValue;
+  if (D != 64 && D != 128) return (int)hipErrorInvalidValue;
+  const long units = gather_units(B, Hq, Hk, per_head);
+  int chunk, ns;
+  gather_plan(kb, units, chunk_req, &chunk, &ns);
+  *bytes = splitk_workspace_bytes(units, ns, D);
+  return 0;
+}
+
+int bytes_gather_attn(const void* q, const void* k, const void* v, int kv_fp8, const void* idx, void* out, int B,
+                      int Hq, int Hk, int S, int D, int kb, int per_head, int page, int limit, int64_t q_sb, int64_t q_sh,
+                      int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss, int64_t i_sb, int64_t i_sh,
+                      int64_t o_sb, int64_t o_sh, float scaling, int chunk_req, void* workspace,
+                      size_t workspace_bytes, void* stream) {
+  return gather_attn(q, k, v, kv_fp8, idx, nullptr, nullptr, 1, out, B, Hq, Hk, S, D, kb, per_head, page, limit, q_sb,
+                     q_sh, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, i_sb, i_sh, o_sb, o_sh, scaling, chunk_req, workspace,
+                     workspace_bytes, stream);
+}
+
+int bytes_attend_topk(const void* q, const void* k, const void* v, int kv_fp8, const void* idx, const void* pos, int Qc,
+                      void* out, int B, int Hq, int Hk, int S, int D, int kb, int64_t q_sb, int64_t q_sh, int64_t k_sb,
+                      int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss, int64_t i_sb, int64_t i_sh,
+                      int64_t o_sb, int64_t o_sh, float scaling, void* workspace, size_t workspace_bytes,
+                      void* stream) {
+  if (!idx || !pos || Qc <= 0) return (int)hipErrorInvalidValue;
+  return gather_attn(q, k, v, kv_fp8, nullptr, idx, pos, Qc, out, B, Hq, Hk, S, D, kb, 1, 0, S, q_sb, q_sh, k_sb, k_sh,
+                     k_ss, v_sb, v_sh, v_ss, i_sb, i_sh, o_sb, o_sh, scaling, 0, workspace, workspace_bytes, stream);
 }
 
 // Quest decode after the page bounds: per query head, the top npick pages of
@@ -361,6 +413,10 @@ int bytes_quest_gather_attn(const void* q, const void* k, const void* v, int kv_
   a.v = v;
   a.v_sb = v_sb; a.v_sh = v_sh; a.v_ss = v_ss;
   a.idx = nullptr;
+  a.idx64 = nullptr;
+  a.pos = nullptr;
+  a.Qc = 1;
+  a.nt = true;
   a.i_sb = a.i_sh = 0;
   a.Hk = Hk; a.G = Hq / Hk; a.HB = (a.G + 15) / 16; a.S = S; a.kb = kb;
   a.per_head = 1;

@@ -683,6 +683,87 @@ __global__ __launch_bounds__(kScoreWaves * 64, 2) void score_kernel(ScoreArgs a)
 
 #pragma clang diagnostic pop
 
+// ---- bf16 keys, many query heads per KV head ------------------------------
+// Per-head scores of folded query chunks (a KV head's group then holds G * Qc
+// heads): a product of [heads x D] and [D x tokens] whose output is the
+// traffic.  A wave holds 64 tokens' keys as A operands in registers and walks
+// the workgroup's blocks of 16 heads, so the keys are read once per head range
+// instead of once per 16 heads; with tokens as MFMA rows a lane receives four
+// consecutive tokens of one head, stored 16 bytes at once.  Operands take the
+// dims of each contraction step as the streaming kernel's do, so the scores
+// are the same bits.  3584 heads x 2048 keys of 64: 18 us in the streaming
+// kernel (one pass over the keys per 16 heads), 13 us here; bound by the stores
+// (29 MB, 64-byte pieces of 16 rows per instruction).
+constexpr int kScoreBlockHeads = 64;   // heads per KV head from which this kernel is taken
+
+struct ScoreBlockArgs {
+  const uint16_t* q;
+  int64_t q_sb, q_sh;
+  const uint16_t* k;
+  int64_t k_sb, k_sh, k_ss;
+  float* out;
+  int64_t o_sb, o_sh;
+  int Hk, G, S, HB, hpw, hgroups, tparts;   // HB blocks of 16 heads, hpw of them per workgroup
+  float scaling;
+};
+
+template <int D>
+__global__ __launch_bounds__(kScoreWaves * 64, 4) void score_block_kernel(ScoreBlockArgs a) {
+  constexpr int KK = D / 32;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, l16 = lane & 15, lg = lane >> 4;
+  int r = blockIdx.x;
+  const int tp = r % a.tparts;
+  r /= a.tparts;
+  const int hg = r % a.hgroups;
+  r /= a.hgroups;
+  const int hk = r % a.Hk, b = r / a.Hk;
+  const int t0 = tp * (kScoreWaves * 64) + w * 64;
+  if (t0 >= a.S) return;                         // wave-uniform, no barrier in this kernel
+  const uint16_t* kb = a.k + (int64_t)b * a.k_sb + (int64_t)hk * a.k_sh + lg * 8;
+  bf16x8 ka[4][KK];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const uint16_t* row = kb + (int64_t)min(t0 + c * 16 + l16, a.S - 1) * a.k_ss;
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) ka[c][kk] = __builtin_bit_cast(bf16x8, ld16(row + kk * 32));
+  }
+  const uint16_t* qb = a.q + (int64_t)b * a.q_sb + (int64_t)hk * a.G * a.q_sh + lg * 8;
+  float* ob = a.out + (int64_t)b * a.o_sb + (int64_t)hk * a.G * a.o_sh + t0;
+  auto fetch = [&](int hb, bf16x8 (&q)[KK]) {
+    const uint16_t* row = qb + (int64_t)min(hb * 16 + l16, a.G - 1) * a.q_sh;
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) q[kk] = __builtin_bit_cast(bf16x8, ld16(row + kk * 32));
+  };
+  const int h_end = min((hg + 1) * a.hpw, a.HB);
+  bf16x8 nxt[KK];
+  fetch(hg * a.hpw, nxt);
+  for (int hb = hg * a.hpw; hb < h_end; ++hb) {
+    bf16x8 q[KK];
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) q[kk] = nxt[kk];
+    fetch(min(hb + 1, h_end - 1), nxt);
+    const int h = hb * 16 + l16;
+    float* o = ob + (int64_t)min(h, a.G - 1) * a.o_sh;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) s = mfma_bf16(ka[c][kk], q[kk], s);
+      s *= a.scaling;
+      const int t = c * 16 + lg * 4;             // from t0
+      if (h < a.G) {
+        if (t0 + t + 4 <= a.S) {
+          *reinterpret_cast<f32x4*>(o + t) = s;
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (t0 + t + i < a.S) o[t + i] = s[i];
+        }
+      }
+    }
+  }
+}
+
 template <int D, bool FP8>
 static void launch_dense(const dim3& g, const dim3& blk, hipStream_t st, const ScoreArgs& a) {
   if (a.group_sum)
@@ -764,6 +845,33 @@ int bytes_sparse_score(const void* q, const void* k, int k_mode, const void* k_s
       ((int64_t)S + 64) * k_ss * (k_mode == kKeyBf16 ? 2 : 1) >= ((int64_t)1 << 32))
     return (int)hipErrorNotSupported;
   a.scaling = scaling;
+  // many heads per KV head (folded query chunks), output rows on 16-byte
+  // boundaries: the block kernel
+  if (k_mode == kKeyBf16 && !a.group_sum && a.G >= kScoreBlockHeads && reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
+      o_sb % 4 == 0 && o_sh % 4 == 0) {
+    ScoreBlockArgs c;
+    c.q = a.q; c.q_sb = q_sb; c.q_sh = q_sh;
+    c.k = static_cast<const uint16_t*>(k);
+    c.k_sb = k_sb; c.k_sh = k_sh; c.k_ss = k_ss;
+    c.out = a.out; c.o_sb = o_sb; c.o_sh = o_sh;
+    c.Hk = Hk; c.G = a.G; c.S = S;
+    c.HB = (a.G + 15) / 16;
+    c.scaling = scaling;
+    c.tparts = (S + kScoreWaves * 64 - 1) / (kScoreWaves * 64);
+    // about four workgroups per CU, so the keys' first loads of some overlap
+    // the stores of others
+    const long blocks = (long)B * Hk * c.tparts * c.HB, want = 4L * device_cu_count();
+    const long hpw = (blocks + want - 1) / want;
+    c.hpw = (int)(hpw < c.HB ? hpw : c.HB);
+    c.hgroups = (c.HB + c.hpw - 1) / c.hpw;
+    const long wgs = (long)B * Hk * c.tparts * c.hgroups;
+    if (wgs > 0x7FFFFFFFL) return (int)hipErrorInvalidConfiguration;
+    const dim3 g2((unsigned)wgs), b2(kScoreWaves * 64);
+    hipStream_t st2 = static_cast<hipStream_t>(stream);
+    if (D == 128) BYTES_LAUNCH(kProfScore, (score_block_kernel<128>), g2, b2, 0, st2, c);
+    else BYTES_LAUNCH(kProfScore, (score_block_kernel<64>), g2, b2, 0, st2, c);
+    return (int)hipGetLastError();
+  }
   const long units = (long)B * Hk * a.HB;
   // about 8 workgroups per CU in total (eight rounds of one resident with
   // 256-byte key rows, four of two otherwise), each a multiple of one

@@ -36,9 +36,9 @@ from __future__ import annotations
 import torch
 
 from . import _checks as C
-from ._lib import call, native, ptr, stream_of
+from ._lib import call, native, ptr, size_query, stream_of, workspace
 from .quest import quest_page_minmax, quest_page_scores
-from .sparse import _score, _topk, sparse_gather_attn, topk_indices
+from .sparse import _qk_shapes, _score, _topk, sparse_gather_attn, topk_indices
 
 # selectors that rank by exact fp32 scores of the keys passed in (the
 # reference's "exact" and its SOFT_SELECTORS other than "signvq", :35, which
@@ -222,6 +222,27 @@ def _quest_select(q_blk, k_r, pos, S, kb, page, scaling, local_w=0):
     return tok
 
 
+def _attend_int64(qf, k, v, idx, pos, Qc: int, scaling: float) -> torch.Tensor:
+    """sparse_gather_attn over int64 lists idx [B, H_q, kb] (contiguous), masked
+    by position as they are read."""
+    B, Hq, Hk, S, D = _qk_shapes(qf, k)
+    C.cuda_tensors(qf, v, idx)
+    C.dtype_in(k, "k", torch.bfloat16, torch.float8_e4m3fn)
+    C.dtype_in(v, "v", k.dtype)
+    if tuple(v.shape) != tuple(k.shape):
+        raise ValueError(f"shape mismatch: k {tuple(k.shape)}, v {tuple(v.shape)}")
+    kb = idx.shape[-1]
+    qs = C.rows16(qf.squeeze(2))
+    k, v = C.rows16(k), C.rows16(v)
+    out = torch.empty((B, Hq, D), dtype=torch.bfloat16, device=qf.device)
+    ws = workspace(qf.device, size_query("bytes_gather_attn_workspace_size", B, Hq, Hk, kb, D, 1, 0))
+    call("bytes_attend_topk", ptr(qs), ptr(k), ptr(v), int(k.dtype == torch.float8_e4m3fn), ptr(idx), ptr(pos), Qc,
+         ptr(out), B, Hq, Hk, S, D, kb, qs.stride(0), qs.stride(1), k.stride(0), k.stride(1), k.stride(2), v.stride(0),
+         v.stride(1), v.stride(2), idx.stride(0), idx.stride(1), out.stride(0), out.stride(1), float(scaling), ptr(ws),
+         ws.numel(), stream_of(qf))
+    return out
+
+
 def attend_topk(q_blk, k_r, v, idx, q_pos, scaling):
     """Exact attention of each query row over its selected keys
     (benchmarks/sparse_attention.py:367-387).
@@ -235,7 +256,10 @@ def attend_topk(q_blk, k_r, v, idx, q_pos, scaling):
         raise ValueError(f"idx must be [B, Hq, Qc, ksel] = [{B}, {Hq}, {Qc}, .]; got {tuple(idx.shape)}")
     C.cuda_tensors(idx)
     pos, _ = _positions(q_pos, Qc, q_blk.device)
-    S = k_r.shape[2]
-    rows = _fill(idx, pos, Qc, S, idx.shape[-1], torch.int32).reshape(B, Hq * Qc, idx.shape[-1])
-    out = sparse_gather_attn(qf, k_r, v, rows, scaling)
+    S, kb = k_r.shape[2], idx.shape[-1]
+    if idx.dtype == torch.int64 and idx.is_contiguous() and kb:
+        out = _attend_int64(qf, k_r, v, idx.view(B, Hq * Qc, kb), pos, Qc, scaling)
+    else:
+        rows = _fill(idx, pos, Qc, S, kb, torch.int32).reshape(B, Hq * Qc, kb)
+        out = sparse_gather_attn(qf, k_r, v, rows, scaling)
     return out.reshape(B, Hq, Qc, D)

@@ -233,6 +233,19 @@ int bytes_gather_attn(const void* q, const void* k, const void* v, int kv_fp8, c
                       int64_t o_sb, int64_t o_sh, float scaling, int chunk, void* workspace,
                       size_t workspace_bytes, void* stream);
 
+/* Attention of a query chunk's rows over their selected keys: replaces
+ * benchmarks/sparse_attention.py:367-387 (`attend_topk`).  bytes_gather_attn
+ * with per_head = 1 over int64 lists idx [B, Hq, kb] as the selection functions
+ * give them, Hq folded as (head, query row): list h belongs to query row
+ * h % Qc, whose position is pos[h % Qc] (int64 device array of Qc entries).
+ * Entries that are negative, >= S or past their row's position take no part.
+ * Workspace: bytes_gather_attn_workspace_size (per_head = 1, chunk = 0). */
+int bytes_attend_topk(const void* q, const void* k, const void* v, int kv_fp8, const void* idx, const void* pos,
+                      int Qc, void* out, int B, int Hq, int Hk, int S, int D, int kb, int64_t q_sb, int64_t q_sh,
+                      int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss,
+                      int64_t i_sb, int64_t i_sh, int64_t o_sb, int64_t o_sh, float scaling, void* workspace,
+                      size_t workspace_bytes, void* stream);
+
 /* ---------------------------------------------------------------------------
  * Quest page metadata and bounds.
  * Replaces the page part of benchmarks/sparse_attention.py:328-364 (`_quest_select`;

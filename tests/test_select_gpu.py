@@ -210,3 +210,28 @@ def test_select_step_sizes(dev, S, kb, k_chunk, local_w):
         s = SP.sparse_score_scalar(q.reshape(B, Hq * Qc, 1, D).to(dev), k.to(dev), 0.125).cpu()
         want = R.select_topk_from_scores(s.reshape(B, Hq, Qc, S), pos, S, kb, k_chunk, local_w)
         assert torch.equal(got.cpu(), want), integer
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+def test_attend_topk_list_dtypes(dev, fp8):
+    """int64 lists are masked as the attention reads them, int32 and strided
+    ones by a launch of their own: the same bits, with entries that are
+    negative, duplicate, past S or past their row's position; lists that hold
+    the cache several times over (plain row loads) and lists that do not."""
+    for S, ksel, Qc in ((96, 200, 5), (3000, 40, 2)):
+        q, k, v = _inputs(1, 6, 2, Qc, S, 64, seed=S)
+        if fp8:
+            k, v = k.to(torch.float8_e4m3fn), v.to(torch.float8_e4m3fn)
+        g = torch.Generator().manual_seed(ksel)
+        idx = torch.randint(-3, S + 9, (1, 6, Qc, ksel), generator=g)
+        idx[0, 0, 0, 0] = 2 ** 40
+        idx[0, 1, 0, 0] = -2 ** 40
+        pos = torch.linspace(S // 2, S - 1, Qc).long()
+        qd, kd, vd, i = q.to(dev), k.to(dev), v.to(dev), idx.to(dev)
+        got = SA.attend_topk(qd, kd, vd, i, pos, 0.125)
+        assert torch.equal(got, SA.attend_topk(qd, kd, vd, i.clamp(-3, S + 9).int(), pos, 0.125))
+        wide = torch.zeros(1, 6, Qc, ksel + 1, dtype=torch.int64, device=dev)
+        wide[..., :ksel] = i
+        assert torch.equal(got, SA.attend_topk(qd, kd, vd, wide[..., :ksel], pos, 0.125))
+        if not fp8:
+            _check(got, R.attend_topk(q, k, v, idx.clamp(-3, S + 9), pos, 0.125), f"attend S {S}")

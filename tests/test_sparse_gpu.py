@@ -384,3 +384,28 @@ def test_token_topk_c5_full(dev, kb):
     gi = idx.long().unsqueeze(-1).expand(B, Hk, kb, k.shape[-1])
     ks, vs = torch.gather(k, 2, gi).cpu(), torch.gather(v, 2, gi).cpu()
     _check(out, R.decode_attn(q.cpu(), ks, vs, scale=sc), f"C5 kb{kb}")
+
+
+@pytest.mark.parametrize("B,Hk,G,S,D", [(1, 2, 64, 257, 64), (2, 1, 65, 1000, 128), (1, 1, 1792, 2047, 64),
+                                        (1, 3, 100, 3, 128)])
+def test_score_many_heads_per_kv_head(dev, B, Hk, G, S, D):
+    """64 or more heads per KV head (folded query chunks) take the block kernel:
+    the same bits as the streaming kernel gives 16 heads at a time, for token
+    counts and head counts that fill no block, into rows of a wider buffer too."""
+    from bytes_amd.sparse import _score
+    g = torch.Generator().manual_seed(S + G)
+    q = torch.randn(B, Hk * G, 1, D, generator=g).to(torch.bfloat16).to(dev)
+    k = torch.randn(B, Hk, S, D, generator=g).to(torch.bfloat16).to(dev)
+    got = SP.sparse_score_scalar(q, k, 0.3)
+    qg = q.reshape(B, Hk, G, 1, D)
+    want = torch.empty(B, Hk, G, S, device=dev)
+    for h0 in range(0, G, 16):
+        n = min(16, G - h0)
+        part = qg[:, :, h0:h0 + n].reshape(B, Hk * n, 1, D)
+        want[:, :, h0:h0 + n] = SP.sparse_score_scalar(part, k, 0.3).reshape(B, Hk, n, S)
+    assert torch.equal(got, want.reshape(B, Hk * G, S))
+    wide = torch.full((B, Hk * G, (S + 7) // 4 * 4), 7.0, device=dev)
+    _score(q, k, 0.3, group_sum=False, out=wide[:, :, 4:4 + S] if wide.shape[2] >= S + 4 else wide[:, :, :S])
+    lo = 4 if wide.shape[2] >= S + 4 else 0
+    assert torch.equal(wide[:, :, lo:lo + S], got)
+    assert (wide[:, :, :lo] == 7).all() and (wide[:, :, lo + S:] == 7).all()
