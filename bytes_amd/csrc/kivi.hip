@@ -254,6 +254,8 @@ struct KiviArgs {
   const uint16_t* vr;
   int64_t kr_sb, kr_sh, kr_ss, vr_sb, vr_sh, vr_ss;
   int Hk, G, HB, Sq, R, chunk, nsq;
+  int nquant;               // pipelined kernel: workgroups of quantized splits
+  FastDiv dsq, drs;         // pipelined kernel: division by nsq and rsplit
   int rsplit;               // > 0: the residual window has splits nsq .. nsq+rsplit-1 of its own (128 tokens each)
   int rchunk;               // rsplit == 0: residual tokens per piece (<= 128; pieces ride on the last splits)
   float scale_log2;
@@ -1393,6 +1395,24 @@ struct PipeMeta {
   u32x4 vm;              // value scales (lanes 0-31) / zeros (32-63) of tokens 2(l % 32), +1 of the wave's tile
 };
 
+// (unit, split) of a workgroup: the residual window's splits come first in the
+// grid, then the quantized splits in the XCDs' runs.  The residual splits are
+// short and the quantized ones alike, so those that fill the CUs' slots once
+// all start early and end together.  With each unit's residual splits after its
+// quantized ones, the quantized splits that these displaced from the first pass
+// started only when others had ended: 4-bit B32 H_k8 L16K, 512 quantized splits
+// on 512 slots, 176 us then and 137 now (129 with no residual window).
+__device__ __forceinline__ UnitLoc pipe_locate(const KiviArgs& a) {
+  const int L = blockIdx.x, nr = a.o.nwg - a.nquant;
+  if (L < nr) {
+    const int unit = fast_div(L, a.drs);
+    return splitk_unit(a.o, unit, a.nsq + L - unit * a.rsplit);
+  }
+  const int idx = xcd_run(L - nr, a.nquant);
+  const int unit = fast_div(idx, a.dsq);
+  return splitk_unit(a.o, unit, idx - unit * a.nsq);
+}
+
 template <int D, int BITS>
 __global__ __launch_bounds__(kPipeWaves * 64, pipe_wg_per_cu<BITS>()) void kivi_pipe_kernel(KiviArgs a) {
   using C = PipeCfg<D, BITS>;
@@ -1401,7 +1421,7 @@ __global__ __launch_bounds__(kPipeWaves * 64, pipe_wg_per_cu<BITS>()) void kivi_
   __shared__ __attribute__((aligned(16))) char st1[C::STAGE];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, lg = lane >> 4;
-  const UnitLoc loc = splitk_locate(a.o);
+  const UnitLoc loc = pipe_locate(a);
   const int unit = loc.unit, split = loc.split, b = loc.b, hk = loc.hk, hb = loc.hb;
   const int hq0 = hk * a.G + hb * 16;
   const int nh = min(16, a.G - hb * 16);
@@ -1621,27 +1641,43 @@ static void kivi_stream_plan(int Sq, int R, long units, int chunk_req, int gran,
   *rchunk = 0;
 }
 
-// Granules per split of the pipelined kernel chosen by the library: the
-// fewest that keep the grid within two workgroups per CU (one pass of the
-// grid, measured best at L = 24K-128K, B4 H_k4, for both bit widths: e.g. 2-bit
-// L32K 22.0 us at four granules against 27.0 at eight, L64K 31.0 at eight
-// against 33.2 at six and 32.5 at ten).
+// Granules per split of the pipelined kernel chosen by the library.  Counted
+// in passes of two workgroups per CU (best for both bit widths, though three
+// 2-bit ones fit: B32 H_k8 L16K 90 us in one pass of two, 109 with three), the
+// splits that fill p = 1..8 passes are compared by passes * (granules per split
+// + 1), the 1 for a workgroup's first loads and its epilogue, and cut evenly:
+// one pass where the units divide the slots well (2-bit B4 H_k4 L64K 30 us at
+// eight granules against 33 at six and 35 at twelve), several where they do
+// not (2-bit B48 H_k8 L16K, 384 units: 148 us at sixteen granules in three
+// passes, 156 with one split of 64 per unit and a quarter of the slots empty,
+// 181 with splits of 48 and 16).
 static int kivi_pipe_gps(int Sq, long units) {
   const long ng = (Sq + kPipeGran - 1) / kPipeGran;
   const long slots = 2L * device_cu_count();
-  return (int)((ng * units + slots - 1) / slots);
+  long best = 0, best_cost = 0;
+  for (int p = 1; p <= 8; ++p) {
+    long n = p * slots / units;
+    n = n < 1 ? 1 : n > ng ? ng : n;
+    const long gps = (ng + n - 1) / n;
+    n = (ng + gps - 1) / gps;
+    const long cost = (n * units + slots - 1) / slots * (gps + 1);
+    if (p == 1 || cost < best_cost) best = gps, best_cost = cost;
+    if (n == ng) break;
+  }
+  return (int)best;
 }
 
 // The pipelined kernel serves D = 128 caches (2- or 4-bit) of whole 64-token
 // tiles and at least four granules: always when the caller asks for it
 // (chunk_req < 0), never when the caller sets a split length for the other
-// kernels (chunk_req > 0), and otherwise when its splits are at least three
-// granules long (B4 H_k4 from L = 24K; shorter caches finish sooner on the
-// two-half kernel, whose splits are shorter).
+// kernels (chunk_req > 0), and otherwise when two workgroups per CU get at
+// least three granules each (B4 H_k4 from L = 24K; shorter caches finish sooner
+// on the two-half kernel, whose splits are shorter).
 static bool kivi_use_pipe(int D, int bits, int Sq, long units, int chunk_req) {
   if (D != 128 || Sq % kKiviTile != 0 || Sq < 4 * kPipeGran) return false;
   if (chunk_req != 0) return chunk_req < 0;
-  return kivi_pipe_gps(Sq, units) >= 3;
+  const long ng = (Sq + kPipeGran - 1) / kPipeGran;
+  return ng * units > 2 * 2L * device_cu_count();
 }
 
 // Plan of the pipelined kernel: the residual window on splits of its own
@@ -1804,6 +1840,9 @@ int bytes_kivi_decode_attn(const void* q, const void* kq, const void* k_scale, c
   hipStream_t st = static_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)(ns * units));
   if (pipe) {
+    a.nquant = (int)(a.nsq * units);
+    a.dsq = make_fastdiv((uint32_t)a.nsq);
+    a.drs = make_fastdiv((uint32_t)(a.rsplit > 0 ? a.rsplit : 1));
     if (bits == 2) BYTES_LAUNCH(kProfKivi, (kivi_pipe_kernel<128, 2>), grid, dim3(kPipeWaves * 64), 0, st, a);
     else BYTES_LAUNCH(kProfKivi, (kivi_pipe_kernel<128, 4>), grid, dim3(kPipeWaves * 64), 0, st, a);
     int rc = (int)hipGetLastError();

@@ -72,21 +72,27 @@ __device__ __forceinline__ void xcd_unit_split(int nsplit, int N, int& unit, int
 struct UnitLoc {
   int unit, split, b, hk, hb;
 };
-__device__ __forceinline__ UnitLoc splitk_locate(const SplitKOut& o) {
-  const int L = blockIdx.x;
+// Position L of N dealt over the XCDs -> its place in the order of (unit, split).
+__device__ __forceinline__ int xcd_run(int L, int N) {
   const int x = L % kXcds, k = L / kXcds;
-  const int q = o.nwg / kXcds, r = o.nwg % kXcds;
-  const int idx = x * q + min(x, r) + k;
+  const int q = N / kXcds, r = N % kXcds;
+  return x * q + min(x, r) + k;
+}
+__device__ __forceinline__ UnitLoc splitk_unit(const SplitKOut& o, int unit, int split) {
   UnitLoc u;
-  u.unit = fast_div(idx, o.dsplit);
-  u.split = idx - u.unit * o.nsplit;
-  u.b = fast_div(u.unit, o.dunit);
-  const int rem = u.unit - u.b * (int)o.dunit.d;
+  u.unit = unit;
+  u.split = split;
+  u.b = fast_div(unit, o.dunit);
+  const int rem = unit - u.b * (int)o.dunit.d;
   u.hk = fast_div(rem, o.dhb);
   u.hb = rem - u.hk * (int)o.dhb.d;
   return u;
 }
-
+__device__ __forceinline__ UnitLoc splitk_locate(const SplitKOut& o) {
+  const int idx = xcd_run(blockIdx.x, o.nwg);
+  const int unit = fast_div(idx, o.dsplit);
+  return splitk_unit(o, unit, idx - unit * o.nsplit);
+}
 
 // Raw buffer resource over [base, base + bytes) (out-of-range lanes read 0 and
 // drop stores).

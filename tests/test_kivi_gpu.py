@@ -245,6 +245,17 @@ def test_decode_pipelined(dev, bits, B, Hq, Hk, L, Rw, gps):
 
 
 @pytest.mark.parametrize("bits", [2, 4])
+@pytest.mark.parametrize("B,Hq,Hk,L,Rw", [
+    (75, 8, 8, 1024 + 1, 1),            # 600 units: more than a pass of one split each, one residual token
+    (48, 16, 8, 1536 + 64 + 129, 129),  # 384 units, two residual splits each, a partial last granule
+    (43, 6, 6, 2048 + 300, 300),        # 258 units, three residual splits each: 774 ahead of the quantized ones
+    (32, 8, 8, 2048, 0),                # no residual window
+])
+def test_decode_pipelined_many_units(dev, bits, B, Hq, Hk, L, Rw):
+    _decode_case(dev, bits, B, Hq, Hk, 128, L, Rw, seed=L + B + bits)
+
+
+@pytest.mark.parametrize("bits", [2, 4])
 def test_decode_pipelined_long_cache_automatic(dev, bits):
     """A long cache (B=4, Hk=4, Sq=32768: four-granule splits fill two
     workgroups per CU) takes the pipelined kernel by default."""
