@@ -251,7 +251,7 @@ Tensor pq_fused(const Tensor& q, const Tensor& kcb, const Tensor& ki, const Tens
   return out;
 }
 
-// LUT + outlier scores, dense values; paged where bt is given.
+// LUT + outlier scores, dense values; paged where bt and cl are given (both or neither).
 Tensor pq_asym(const Tensor& lut, const Tensor& ki, const Tensor& ko, const Tensor& qo, const Tensor& v,
                const Tensor* bt, const Tensor* cl, long block_size, long chunk) {
   need(lut.dim() == 4 && ki.dim() == 4 && ko.dim() == 4 && qo.dim() == 3 && lut.scalar_type() == at::kFloat);
@@ -518,8 +518,10 @@ BIND(kivi, 13, (need(integer(a[10]) == 32),
 BIND(kivi_pack, 3, kivi_pack(tensor(a[0]), integer(a[1]), integer(a[2])))
 BIND(pq_fused, 7, WRAP(pq_fused(tensor(a[0]), tensor(a[1]), tensor(a[2]), tensor(a[3]), tensor(a[4]), number(a[5]),
                                 integer(a[6]))))
-BIND(pq_asym, 9, WRAP(pq_asym(tensor(a[0]), tensor(a[1]), tensor(a[2]), tensor(a[3]), tensor(a[4]), optional(a[5]),
-                              optional(a[6]), integer(a[7]), integer(a[8]))))
+BIND(pq_asym, 6, WRAP(pq_asym(tensor(a[0]), tensor(a[1]), tensor(a[2]), tensor(a[3]), tensor(a[4]), nullptr, nullptr, 0,
+                              integer(a[5]))))
+BIND(pq_paged, 9, WRAP(pq_asym(tensor(a[0]), tensor(a[1]), tensor(a[2]), tensor(a[3]), tensor(a[4]), &tensor(a[5]),
+                               &tensor(a[6]), integer(a[7]), integer(a[8]))))
 BIND(pq_encode, 2, WRAP(pq_encode(tensor(a[0]), tensor(a[1]))))
 BIND(score_into, 4, (score_into(tensor(a[0]), tensor(a[1]), nullptr, nullptr, 0, number(a[2]), false, tensor(a[3]), nullptr),
                      Py_NewRef(a[3])))
@@ -545,7 +547,7 @@ PyObject* py_set_workspaces(PyObject*, PyObject* d) {
 
 #define METHOD(NAME) {#NAME, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_##NAME)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {METHOD(dense),     METHOD(kivi),   METHOD(kivi_pack), METHOD(pq_fused),
-                         METHOD(pq_asym),   METHOD(pq_encode), METHOD(score_into), METHOD(topk),
+                         METHOD(pq_asym),   METHOD(pq_paged), METHOD(pq_encode), METHOD(score_into), METHOD(topk),
                          METHOD(gather),    METHOD(sparse_decode), METHOD(token_topk), METHOD(quest),
                          {"set_workspaces", py_set_workspaces, METH_O, nullptr},
                          {nullptr, nullptr, 0, nullptr}};

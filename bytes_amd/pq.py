@@ -275,7 +275,7 @@ def decode_attn_pq_lut_asym(lut: torch.Tensor, k_idx: torch.Tensor, k_out: torch
     k_out [B,H_k,S,C] and q_out [B,H_q,C] (C <= 16; C = 0 allowed); v
     [B,H_k,S,D] bf16 or float8_e4m3fn.  Returns [B,H_q,1,D] in v's dtype, bf16
     for fp8 values (:735)."""
-    out = native().pq_asym(lut, k_idx, k_out, q_out, v, None, None, 0, chunk)
+    out = native().pq_asym(lut, k_idx, k_out, q_out, v, chunk)
     if out is not None:
         return out
     lut, B, Hq, Hk, S, M, K = _lut_checks(lut, k_idx)
@@ -337,7 +337,8 @@ def paged_attn_pq_lut_asym(lut: torch.Tensor, k_idx_paged: torch.Tensor, k_out_p
     k_out_paged [num_blocks,H_k,block_size,C], v_paged [num_blocks,H_k,block_size,D]
     bf16 or float8_e4m3fn, q_out [B,H_q,C].  Returns [B,H_q,1,D] in v's dtype,
     bf16 for fp8 values."""
-    out = native().pq_asym(lut, k_idx_paged, k_out_paged, q_out, v_paged, block_table, context_lens, block_size, chunk)
+    out = native().pq_paged(lut, k_idx_paged, k_out_paged, q_out, v_paged, block_table, context_lens, block_size,
+                            chunk)
     if out is not None:
         return out
     lut, B, Hq, Hk, nblk, bs, M, K = _paged_lut_checks(lut, k_idx_paged)

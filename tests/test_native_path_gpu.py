@@ -135,6 +135,11 @@ def test_pq(dev, monkeypatch):
     _both(monkeypatch, PQ.paged_attn_pq_lut_asym, lut, kp, kop, qo, vp, bt.long(), cl, bs, taken=False)
     with pytest.raises(ValueError):
         PQ.paged_attn_pq_lut_asym(lut, kp, kop, qo, vp, bt, cl, 32)
+    with pytest.raises(ValueError):                                             # as many blocks as sequences
+        PQ.paged_attn_pq_lut_asym(lut, kp[:B], kop[:B], qo, vp[:B], None, None, bs)
+    for tables in ((bt, None), (None, cl)):
+        with pytest.raises(ValueError):
+            PQ.paged_attn_pq_lut_asym(lut, kp, kop, qo, vp, *tables, bs)
     cb = torch.randn(3, M, K, 8, generator=g, device=dev)
     x = torch.randn(3, 2, 77, D, generator=g, device=dev)
     for dt in (torch.float32, torch.bfloat16, torch.float16):
