@@ -261,9 +261,6 @@ def dtype_code(t: torch.Tensor) -> int:
     return codes[t.dtype]
 
 
-HIP_ERROR_NOT_SUPPORTED = 801
-
-
 def size_query(name: str, *args) -> int:
     out = ctypes.c_size_t(0)
     call(name, *args, ctypes.byref(out))
