@@ -393,10 +393,12 @@ const Tensor& gather_workspace(const Tensor& q, const QK& s, int64_t kb, bool pe
   return workspace(q, "splitk", n);
 }
 
+// limit -1: every row.
 Tensor gather(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& idx, double scaling, long chunk,
               long page, long limit) {
   const Kv x = kv(q, k, v);
   const QK& s = x.s;
+  if (limit == -1) limit = s.S;
   need(idx.dim() == 3 && idx.size(0) == s.B && (idx.size(1) == s.Hq || idx.size(1) == s.Hk) && idx.size(2) > 0 &&
        idx.scalar_type() == at::kInt && idx.stride(2) == 1 && page >= 1);
   need(limit >= 0 && limit <= s.S);
@@ -432,7 +434,7 @@ Tensor sparse_decode(const Tensor& q, const Tensor& ks, const Tensor* sc, const 
   gather_workspace(q, s, kb, true, 0);
   Tensor scores = empty(q, {s.B, s.Hq, s.S}, at::kFloat);
   score_into(q, ks, sc, zr, bits, scaling, false, scores, nullptr);
-  return gather(q, k, v, topk_of(scores, kb, false, false), scaling, 0, 1, s.S);
+  return gather(q, k, v, topk_of(scores, kb, false, false), scaling, 0, 1, -1);
 }
 
 PyObject* token_topk(const Tensor& q, const Tensor& k, const Tensor& v, long kb, double scaling, const Tensor& ks,
@@ -448,7 +450,7 @@ PyObject* token_topk(const Tensor& q, const Tensor& k, const Tensor& v, long kb,
   Tensor scores = empty(q, {s.B, s.Hk, s.S}, at::kFloat);
   score_into(q, ks, sc, zr, bits, scaling, true, scores, hist ? w.mutable_data_ptr() : nullptr);
   Tensor idx = topk_of(scores, kb, false, hist);
-  Tensor out = gather(q, k, v, idx, scaling, 0, 1, s.S);
+  Tensor out = gather(q, k, v, idx, scaling, 0, 1, -1);
   return Py_BuildValue("(NN)", THPVariable_Wrap(out), THPVariable_Wrap(idx));
 }
 
@@ -499,6 +501,12 @@ PyObject* guarded(F f) {
   return nullptr;
 }
 
+long row_limit(PyObject* o) {
+  const long v = integer(o);
+  need(v >= 0);
+  return v;
+}
+
 const Tensor* optional(PyObject* o) { return o == Py_None ? nullptr : &tensor(o); }
 
 #define BIND(NAME, N, EXPR)                                                                     \
@@ -527,7 +535,7 @@ BIND(score_into, 4, (score_into(tensor(a[0]), tensor(a[1]), nullptr, nullptr, 0,
                      Py_NewRef(a[3])))
 BIND(topk, 3, WRAP(topk_of(tensor(a[0]), integer(a[1]), a[2] == Py_True, false)))
 BIND(gather, 8, WRAP(gather(tensor(a[0]), tensor(a[1]), tensor(a[2]), tensor(a[3]), number(a[4]), integer(a[5]),
-                            integer(a[6]), a[7] == Py_None ? (long)tensor(a[1]).size(2) : integer(a[7]))))
+                            integer(a[6]), a[7] == Py_None ? -1 : row_limit(a[7]))))
 BIND(sparse_decode, 9, WRAP(sparse_decode(tensor(a[0]), tensor(a[1]), optional(a[2]), optional(a[3]), tensor(a[4]),
                                           tensor(a[5]), number(a[6]), number(a[7]), integer(a[8]))))
 BIND(token_topk, 9, token_topk(tensor(a[0]), tensor(a[1]), tensor(a[2]), integer(a[3]), number(a[4]), tensor(a[5]),

@@ -207,3 +207,13 @@ def test_first_call_and_other_streams(dev, monkeypatch):
         got = _lib.native().dense(q, k2, v, 0.5, 0, False)
     st.synchronize()
     assert torch.equal(got, want)
+
+
+def test_gather_refuses_keys_of_other_ranks(dev):
+    """With no limit given, keys that are not [B, Hk, S, D] are refused as
+    they are with one."""
+    q, k, v = _qkv(dev, 1, 4, 2, 100, 64)
+    idx = torch.zeros(1, 4, 3, dtype=torch.int32, device=dev)
+    for bad in (k[0, 0], k[0, 0, 0]):
+        with pytest.raises(ValueError, match="expected 4 dims"):
+            SP.sparse_gather_attn(q, bad, bad, idx, 0.1)
