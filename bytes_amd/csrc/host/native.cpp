@@ -39,14 +39,17 @@ inline void need(bool ok) {
 
 // A plain CUDA tensor: no subclass, no functorch / functional / Python-key
 // wrapper, no lazy negation or conjugation.
-const Tensor& tensor(PyObject* o) {
-  need(THPVariable_CheckExact(o));
-  const Tensor& t = THPVariable_Unpack(o);
+const Tensor& plain(const Tensor& t) {
   using K = c10::DispatchKey;
   static const c10::DispatchKeySet bad({K::Python, K::PythonTLSSnapshot, K::FuncTorchBatched, K::FuncTorchGradWrapper,
                                         K::Batched, K::Functionalize, K::Negative, K::Conjugate, K::ZeroTensor});
   need(t.defined() && t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has_any(bad) && t.has_storage());
   return t;
+}
+
+const Tensor& tensor(PyObject* o) {
+  need(THPVariable_CheckExact(o));
+  return plain(THPVariable_Unpack(o));
 }
 
 long integer(PyObject* o) {
@@ -88,14 +91,21 @@ const Tensor& workspace(const Tensor& t, const char* family, size_t n) {
   need(key != nullptr);
   PyObject* o = PyDict_GetItem(g_ws, key);       // borrowed; the table keeps every buffer it ever held
   Py_DECREF(key);
-  need(o && THPVariable_CheckExact(o));
-  const Tensor& w = THPVariable_Unpack(o);
+  need(o != nullptr);
+  const Tensor& w = tensor(o);
   need((size_t)w.numel() >= n);
   return w;
 }
 
+// A new tensor on like's device.  Under a dispatch mode it may be one without
+// memory, which the Python wrapper reports.
+Tensor empty(const Tensor& like, at::IntArrayRef s, at::ScalarType dt) {
+  Tensor t = at::empty(s, at::TensorOptions().dtype(dt).device(like.device()));
+  plain(t);
+  return t;
+}
 Tensor empty(const Tensor& like, std::initializer_list<int64_t> s, at::ScalarType dt) {
-  return at::empty(at::IntArrayRef(s), at::TensorOptions().dtype(dt).device(like.device()));
+  return empty(like, at::IntArrayRef(s), dt);
 }
 
 struct Failed {
@@ -103,10 +113,13 @@ struct Failed {
   const char* name;
 };
 
-template <class F>
-void launch(const char* name, F f) {
+// Calls the library without the GIL.  The arguments are evaluated before it is
+// released (a tensor's data pointer may throw), and the library's C functions
+// do not throw.
+template <class... P, class... A>
+void launch(const char* name, int (*f)(P...), A... args) {
   int rc;
-  Py_BEGIN_ALLOW_THREADS rc = f();
+  Py_BEGIN_ALLOW_THREADS rc = f(args...);
   Py_END_ALLOW_THREADS if (rc) throw Failed{rc, name};
 }
 
@@ -149,12 +162,10 @@ Tensor dense(const Tensor& q, const Tensor& k, const Tensor& v, double scale, lo
   const Tensor& w = workspace(q, "splitk", n);
   Tensor out = empty(q, {s.B, s.Hq, 1, s.D}, at::kBFloat16);
   void* st = stream_of(q);
-  launch(fp8 ? "bytes_decode_attn_fp8" : "bytes_decode_attn_bf16", [&] {
-    return (fp8 ? bytes_decode_attn_fp8 : bytes_decode_attn_bf16)(
-        data(q), data(k), data(v), out.mutable_data_ptr(), s.B, s.Hq, s.Hk, s.S, s.D, q.stride(0), q.stride(1),
-        k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2), out.stride(0), out.stride(1),
-        (float)scale, (int)chunk, w.mutable_data_ptr(), (size_t)w.numel(), st);
-  });
+  launch(fp8 ? "bytes_decode_attn_fp8" : "bytes_decode_attn_bf16", fp8 ? bytes_decode_attn_fp8 : bytes_decode_attn_bf16,
+         data(q), data(k), data(v), out.mutable_data_ptr(), s.B, s.Hq, s.Hk, s.S, s.D, q.stride(0), q.stride(1),
+         k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2), out.stride(0), out.stride(1),
+         (float)scale, (int)chunk, w.mutable_data_ptr(), (size_t)w.numel(), st);
   return out;
 }
 
@@ -181,13 +192,11 @@ Tensor kivi(const Tensor& q, const Tensor& kq, const Tensor& ks, const Tensor& k
   Tensor out = empty(q, {B, Hq, 1, D}, at::kBFloat16);
   const float sc = (float)(own_scale ? scale : 1.0 / std::sqrt((double)D));
   void* st = stream_of(q);
-  launch("bytes_kivi_decode_attn", [&] {
-    return bytes_kivi_decode_attn(data(q), data(kq), data(ks), data(km), R ? data(kr) : nullptr, data(vq), data(vs),
-                                  data(vm), R ? data(vr) : nullptr, out.mutable_data_ptr(), B, Hq, Hk, Sq, R, D, bits,
-                                  q.stride(0), q.stride(1), kr.stride(0), kr.stride(1), kr.stride(2), vr.stride(0),
-                                  vr.stride(1), vr.stride(2), out.stride(0), out.stride(1), sc, (int)chunk,
-                                  w.mutable_data_ptr(), (size_t)w.numel(), st);
-  });
+  launch("bytes_kivi_decode_attn", bytes_kivi_decode_attn, data(q), data(kq), data(ks), data(km),
+         R ? data(kr) : nullptr, data(vq), data(vs), data(vm), R ? data(vr) : nullptr, out.mutable_data_ptr(), B, Hq,
+         Hk, Sq, R, D, bits, q.stride(0), q.stride(1), kr.stride(0), kr.stride(1), kr.stride(2), vr.stride(0),
+         vr.stride(1), vr.stride(2), out.stride(0), out.stride(1), sc, (int)chunk, w.mutable_data_ptr(),
+         (size_t)w.numel(), st);
   return out;
 }
 
@@ -198,15 +207,12 @@ PyObject* kivi_pack(const Tensor& x, long group, long bits) {
   const int dt = dtype_code(x);
   auto lead = x.sizes().vec();
   lead.back() = T / fpi;
-  const auto opt = at::TensorOptions().device(x.device());
-  Tensor code = at::empty(lead, opt.dtype(at::kInt));
+  Tensor code = empty(x, lead, at::kInt);
   lead.back() = T / group;
-  Tensor scale = at::empty(lead, opt.dtype(at::kHalf)), mn = at::empty(lead, opt.dtype(at::kHalf));
+  Tensor scale = empty(x, lead, at::kHalf), mn = empty(x, lead, at::kHalf);
   void* st = stream_of(x);
-  launch("bytes_kivi_quantize_pack", [&] {
-    return bytes_kivi_quantize_pack(data(x), dt, x.numel() / T, T, T, group, bits, code.mutable_data_ptr(),
-                                    scale.mutable_data_ptr(), mn.mutable_data_ptr(), st);
-  });
+  launch("bytes_kivi_quantize_pack", bytes_kivi_quantize_pack, data(x), dt, x.numel() / T, T, T, group, bits,
+         code.mutable_data_ptr(), scale.mutable_data_ptr(), mn.mutable_data_ptr(), st);
   return Py_BuildValue("(NNN)", THPVariable_Wrap(code), THPVariable_Wrap(scale), THPVariable_Wrap(mn));
 }
 
@@ -241,13 +247,10 @@ Tensor pq_fused(const Tensor& q, const Tensor& kcb, const Tensor& ki, const Tens
   const Tensor& w = workspace(q, "splitk", n);
   Tensor out = empty(q, {B, Hq, 1, D}, at::kHalf);         // the value codebook's dtype
   void* st = stream_of(q);
-  launch("bytes_pq_decode_attn", [&] {
-    return bytes_pq_decode_attn(3, nullptr, data(q), data(kcb), data(ki), data(vi), data(vcb), nullptr,
-                                out.mutable_data_ptr(), 1, B, Hq, Hk, S, D, k.K, 0, 0, q.stride(0), q.stride(1), k.sh,
-                                ki.stride(0), ki.stride(1), ki.stride(2), vi.stride(0), vi.stride(1), vi.stride(2),
-                                v.sh, 0, 0, 0, out.stride(0), out.stride(1), (float)scale, (int)chunk,
-                                w.mutable_data_ptr(), (size_t)w.numel(), st);
-  });
+  launch("bytes_pq_decode_attn", bytes_pq_decode_attn, 3, nullptr, data(q), data(kcb), data(ki), data(vi), data(vcb),
+         nullptr, out.mutable_data_ptr(), 1, B, Hq, Hk, S, D, k.K, 0, 0, q.stride(0), q.stride(1), k.sh, ki.stride(0),
+         ki.stride(1), ki.stride(2), vi.stride(0), vi.stride(1), vi.stride(2), v.sh, 0, 0, 0, out.stride(0),
+         out.stride(1), (float)scale, (int)chunk, w.mutable_data_ptr(), (size_t)w.numel(), st);
   return out;
 }
 
@@ -282,15 +285,13 @@ Tensor pq_asym(const Tensor& lut, const Tensor& ki, const Tensor& ko, const Tens
   const int kd = dtype_code(ko), qd = dtype_code(qo);
   Tensor out = empty(lut, {B, Hq, 1, D}, at::kBFloat16);
   void* st = stream_of(lut);
-  launch("bytes_pq_lut_decode_attn", [&] {
-    return bytes_pq_lut_decode_attn(
-        data(lut), lut.stride(0), lut.stride(1), data(ki), ki.stride(0), ki.stride(1), ki.stride(2), nullptr, 0, 0, 0,
-        nullptr, 0, data(v), f8, v.stride(0), v.stride(1), v.stride(2), data(ko), kd, ko.stride(0), ko.stride(1),
-        ko.stride(2), data(qo), qd, qo.stride(0), qo.stride(1), (int)C, bt ? bt->const_data_ptr<int>() : nullptr,
-        bt ? bt->stride(0) : 0, cl ? cl->const_data_ptr<int>() : nullptr, bt ? (int)bs : 0, bt ? (int)lead : 0,
-        out.mutable_data_ptr(), 0, out.stride(0), out.stride(1), B, Hq, Hk, S, D, K, 1.0f, (int)chunk,
-        w.mutable_data_ptr(), (size_t)w.numel(), st);
-  });
+  launch("bytes_pq_lut_decode_attn", bytes_pq_lut_decode_attn, data(lut), lut.stride(0), lut.stride(1), data(ki),
+         ki.stride(0), ki.stride(1), ki.stride(2), nullptr, 0, 0, 0, nullptr, 0, data(v), f8, v.stride(0), v.stride(1),
+         v.stride(2), data(ko), kd, ko.stride(0), ko.stride(1), ko.stride(2), data(qo), qd, qo.stride(0), qo.stride(1),
+         (int)C, bt ? bt->const_data_ptr<int>() : nullptr, bt ? bt->stride(0) : 0,
+         cl ? cl->const_data_ptr<int>() : nullptr, bt ? (int)bs : 0, bt ? (int)lead : 0, out.mutable_data_ptr(), 0,
+         out.stride(0), out.stride(1), B, Hq, Hk, S, D, K, 1.0f, (int)chunk, w.mutable_data_ptr(), (size_t)w.numel(),
+         st);
   return out;
 }
 
@@ -305,12 +306,10 @@ Tensor pq_encode(const Tensor& x, const Tensor& cb) {
   auto s = x.sizes().vec();
   s.back() = M;
   const int64_t n = x.numel() / D;
-  Tensor idx = at::empty(s, at::TensorOptions().dtype(at::kByte).device(x.device()));
+  Tensor idx = empty(x, s, at::kByte);
   void* st = stream_of(x);
-  launch("bytes_pq_encode", [&] {
-    return bytes_pq_encode(data(x), xd, heads, n / heads, D, D, data(cb), f32, cb.dim() == 4 ? M * K * 8 : 0, K,
-                           idx.mutable_data_ptr(), st);
-  });
+  launch("bytes_pq_encode", bytes_pq_encode, data(x), xd, heads, n / heads, D, D, data(cb), f32,
+         cb.dim() == 4 ? M * K * 8 : 0, K, idx.mutable_data_ptr(), st);
   return idx;
 }
 
@@ -342,12 +341,10 @@ void score_into(const Tensor& q, const Tensor& k, const Tensor* sc, const Tensor
   need(!group_sum || s.Hq / s.Hk <= 16);
   need(out.scalar_type() == at::kFloat && shape(out, {s.B, group_sum ? s.Hk : s.Hq, s.S}) && out.stride(2) == 1);
   void* st = stream_of(q);
-  launch("bytes_sparse_score", [&] {
-    return bytes_sparse_score(data(q), data(k), mode, packed ? data(*sc) : nullptr, packed ? data(*zr) : nullptr,
-                              out.mutable_data_ptr(), s.B, s.Hq, s.Hk, s.S, s.D, group_sum, q.stride(0), q.stride(1),
-                              k.stride(0), k.stride(1), k.stride(2), m0, m1, m2, out.stride(0), out.stride(1),
-                              (float)scaling, hist, st);
-  });
+  launch("bytes_sparse_score", bytes_sparse_score, data(q), data(k), mode, packed ? data(*sc) : nullptr,
+         packed ? data(*zr) : nullptr, out.mutable_data_ptr(), s.B, s.Hq, s.Hk, s.S, s.D, group_sum, q.stride(0),
+         q.stride(1), k.stride(0), k.stride(1), k.stride(2), m0, m1, m2, out.stride(0), out.stride(1), (float)scaling,
+         hist, st);
 }
 
 const Tensor& topk_workspace(const Tensor& t, int64_t rows_, int64_t n, int64_t k) {
@@ -363,12 +360,10 @@ Tensor topk_of(const Tensor& s, long k, bool sorted, bool hist_ready) {      // 
   const Tensor& w = topk_workspace(s, r, n, k);
   auto shp = s.sizes().vec();
   shp.back() = k;
-  Tensor out = at::empty(shp, at::TensorOptions().dtype(at::kInt).device(s.device()));
+  Tensor out = empty(s, shp, at::kInt);
   void* st = stream_of(s);
-  launch("bytes_topk", [&] {
-    return bytes_topk(data(s), r, (int)n, n, (int)k, sorted, hist_ready, out.mutable_data_ptr(), k,
-                      w.mutable_data_ptr(), (size_t)w.numel(), st);
-  });
+  launch("bytes_topk", bytes_topk, data(s), r, (int)n, n, (int)k, sorted, hist_ready, out.mutable_data_ptr(), k,
+         w.mutable_data_ptr(), (size_t)w.numel(), st);
   return out;
 }
 
@@ -408,13 +403,10 @@ Tensor gather(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& i
   const Tensor& w = gather_workspace(q, s, kb, per_head, chunk);
   Tensor out = empty(q, {s.B, s.Hq, 1, s.D}, at::kBFloat16);
   void* st = stream_of(q);
-  launch("bytes_gather_attn", [&] {
-    return bytes_gather_attn(data(q), data(k), data(v), x.f8, data(idx), out.mutable_data_ptr(), s.B, s.Hq, s.Hk, s.S,
-                             s.D, (int)kb, per_head, page == 1 ? 0 : (int)page, (int)limit, q.stride(0), q.stride(1),
-                             k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2),
-                             idx.stride(0), idx.stride(1), out.stride(0), out.stride(1), (float)scaling, (int)chunk,
-                             w.mutable_data_ptr(), (size_t)w.numel(), st);
-  });
+  launch("bytes_gather_attn", bytes_gather_attn, data(q), data(k), data(v), x.f8, data(idx), out.mutable_data_ptr(),
+         s.B, s.Hq, s.Hk, s.S, s.D, (int)kb, per_head, page == 1 ? 0 : (int)page, (int)limit, q.stride(0), q.stride(1),
+         k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2), idx.stride(0), idx.stride(1),
+         out.stride(0), out.stride(1), (float)scaling, (int)chunk, w.mutable_data_ptr(), (size_t)w.numel(), st);
   return out;
 }
 
@@ -469,18 +461,14 @@ Tensor quest(const Tensor& q, const Tensor& k, const Tensor& v, long kb, double 
   Tensor bound = empty(q, {s.B, s.Hq, np}, at::kFloat);
   Tensor out = empty(q, {s.B, s.Hq, 1, s.D}, at::kBFloat16);
   void* st = stream_of(q);
-  launch("bytes_quest_page_scores", [&] {
-    return bytes_quest_page_scores(data(q), data(kmin), data(kmax), bound.mutable_data_ptr(), s.B, s.Hq, s.Hk, (int)np,
-                                   s.D, (int)page, (int)pos, (int)local_w, q.stride(0), q.stride(1), bound.stride(0),
-                                   bound.stride(1), (float)scaling, st);
-  });
-  launch("bytes_quest_gather_attn", [&] {
-    return bytes_quest_gather_attn(data(q), data(k), data(v), x.f8, data(bound), bound.stride(0), bound.stride(1),
-                                   (int)np, (int)npick, out.mutable_data_ptr(), s.B, s.Hq, s.Hk, s.S, s.D, (int)page,
-                                   (int)pos + 1, q.stride(0), q.stride(1), k.stride(0), k.stride(1), k.stride(2),
-                                   v.stride(0), v.stride(1), v.stride(2), out.stride(0), out.stride(1), (float)scaling,
-                                   0, w.mutable_data_ptr(), (size_t)w.numel(), st);
-  });
+  launch("bytes_quest_page_scores", bytes_quest_page_scores, data(q), data(kmin), data(kmax), bound.mutable_data_ptr(),
+         s.B, s.Hq, s.Hk, (int)np, s.D, (int)page, (int)pos, (int)local_w, q.stride(0), q.stride(1), bound.stride(0),
+         bound.stride(1), (float)scaling, st);
+  launch("bytes_quest_gather_attn", bytes_quest_gather_attn, data(q), data(k), data(v), x.f8, data(bound),
+         bound.stride(0), bound.stride(1), (int)np, (int)npick, out.mutable_data_ptr(), s.B, s.Hq, s.Hk, s.S, s.D,
+         (int)page, (int)pos + 1, q.stride(0), q.stride(1), k.stride(0), k.stride(1), k.stride(2), v.stride(0),
+         v.stride(1), v.stride(2), out.stride(0), out.stride(1), (float)scaling, 0, w.mutable_data_ptr(),
+         (size_t)w.numel(), st);
   return out;
 }
 

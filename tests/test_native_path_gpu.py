@@ -217,3 +217,29 @@ def test_gather_refuses_keys_of_other_ranks(dev):
     for bad in (k[0, 0], k[0, 0, 0]):
         with pytest.raises(ValueError, match="expected 4 dims"):
             SP.sparse_gather_attn(q, bad, bad, idx, 0.1)
+
+
+def test_dispatch_mode_without_storage_is_refused(dev):
+    """Under a mode whose allocations have no memory to point to, a call raises
+    before anything is launched, and the next call outside it works."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class NoMemory(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            if func is torch.ops.aten.empty.memory_format:
+                return torch.sparse_coo_tensor(size=args[0], dtype=kwargs.get("dtype"), device=dev)
+            return func(*args, **(kwargs or {}))
+
+    q, k, v = _qkv(dev, 1, 4, 2, 1000, 64)
+    x = torch.randn(3, 64, device=dev)
+    s = torch.randn(3, 640, device=dev)
+    want = AK.decode_attn_bf16(q, k, v), SP.topk_indices(s, 5)
+    n = _lib.native()
+    with NoMemory():
+        assert n.dense(q, k, v, 1.0, 0, False) is None
+        assert n.kivi_pack(x, 32, 2) is None
+        assert n.topk(s, 5, True) is None
+        assert n.token_topk(q, k, v, 5, 0.1, k, None, None, None) is None
+        with pytest.raises(RuntimeError):
+            AK.decode_attn_bf16(q, k, v)
+    assert torch.equal(AK.decode_attn_bf16(q, k, v), want[0]) and torch.equal(SP.topk_indices(s, 5), want[1])
