@@ -85,14 +85,15 @@ void rows(const Tensor& t, int align = 16) {
 
 void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
-// The family's workspace of the tensor's device, at least n bytes.
-const Tensor& workspace(const Tensor& t, const char* family, size_t n) {
+// The family's workspace of the tensor's device, at least n bytes (held by the
+// caller: another thread may replace the table's entry while the GIL is out).
+Tensor workspace(const Tensor& t, const char* family, size_t n) {
   PyObject* key = Py_BuildValue("(is)", (int)t.device().index(), family);
   need(key != nullptr);
   PyObject* o = PyDict_GetItem(g_ws, key);       // borrowed; the table keeps every buffer it ever held
   Py_DECREF(key);
   need(o != nullptr);
-  const Tensor& w = tensor(o);
+  Tensor w = tensor(o);
   need((size_t)w.numel() >= n);
   return w;
 }
@@ -159,7 +160,7 @@ Tensor dense(const Tensor& q, const Tensor& k, const Tensor& v, double scale, lo
   rows(v);
   size_t n = 0;
   need(bytes_decode_attn_bf16_workspace_size(s.B, s.Hq, s.Hk, s.S, s.D, chunk, &n) == 0);
-  const Tensor& w = workspace(q, "splitk", n);
+  const Tensor w = workspace(q, "splitk", n);
   Tensor out = empty(q, {s.B, s.Hq, 1, s.D}, at::kBFloat16);
   void* st = stream_of(q);
   launch(fp8 ? "bytes_decode_attn_fp8" : "bytes_decode_attn_bf16", fp8 ? bytes_decode_attn_fp8 : bytes_decode_attn_bf16,
@@ -188,7 +189,7 @@ Tensor kivi(const Tensor& q, const Tensor& kq, const Tensor& ks, const Tensor& k
   rows(vr);
   size_t n = 0;
   need(bytes_kivi_decode_workspace_size(B, Hq, Hk, Sq, R, D, bits, chunk, &n) == 0);
-  const Tensor& w = workspace(q, "splitk", n);
+  const Tensor w = workspace(q, "splitk", n);
   Tensor out = empty(q, {B, Hq, 1, D}, at::kBFloat16);
   const float sc = (float)(own_scale ? scale : 1.0 / std::sqrt((double)D));
   void* st = stream_of(q);
@@ -244,7 +245,7 @@ Tensor pq_fused(const Tensor& q, const Tensor& kcb, const Tensor& ki, const Tens
   rows(q);
   size_t n = 0;
   need(bytes_pq_decode_workspace_size(B, Hq, Hk, S, D, chunk, &n) == 0);
-  const Tensor& w = workspace(q, "splitk", n);
+  const Tensor w = workspace(q, "splitk", n);
   Tensor out = empty(q, {B, Hq, 1, D}, at::kHalf);         // the value codebook's dtype
   void* st = stream_of(q);
   launch("bytes_pq_decode_attn", bytes_pq_decode_attn, 3, nullptr, data(q), data(kcb), data(ki), data(vi), data(vcb),
@@ -281,7 +282,7 @@ Tensor pq_asym(const Tensor& lut, const Tensor& ki, const Tensor& ko, const Tens
   need(S > 0 && S <= 0x7FFFFFFF);
   size_t n = 0;
   need(bytes_pq_decode_workspace_size(B, Hq, Hk, S, D, chunk, &n) == 0);
-  const Tensor& w = workspace(lut, "splitk", n);
+  const Tensor w = workspace(lut, "splitk", n);
   const int kd = dtype_code(ko), qd = dtype_code(qo);
   Tensor out = empty(lut, {B, Hq, 1, D}, at::kBFloat16);
   void* st = stream_of(lut);
@@ -347,22 +348,24 @@ void score_into(const Tensor& q, const Tensor& k, const Tensor* sc, const Tensor
          hist, st);
 }
 
-const Tensor& topk_workspace(const Tensor& t, int64_t rows_, int64_t n, int64_t k) {
+Tensor topk_workspace(const Tensor& t, int64_t rows_, int64_t n, int64_t k) {
   size_t bytes = 0;
   need(bytes_topk_workspace_size(rows_, (int)n, (int)k, &bytes) == 0);
   return workspace(t, "topk", bytes);
 }
 
-Tensor topk_of(const Tensor& s, long k, bool sorted, bool hist_ready) {      // contiguous fp32 [.., n]
+// Contiguous fp32 scores [.., n].  counted: the workspace whose histogram region
+// the score kernel has counted them into.
+Tensor topk_of(const Tensor& s, long k, bool sorted, const Tensor* counted) {
   need(s.scalar_type() == at::kFloat && s.dim() >= 1 && s.is_contiguous() && s.numel() > 0);
   const int64_t n = s.size(-1), r = s.numel() / n;
   need(k >= 1 && k <= n && n <= 0x7FFFFFFF);
-  const Tensor& w = topk_workspace(s, r, n, k);
+  const Tensor w = counted ? *counted : topk_workspace(s, r, n, k);
   auto shp = s.sizes().vec();
   shp.back() = k;
   Tensor out = empty(s, shp, at::kInt);
   void* st = stream_of(s);
-  launch("bytes_topk", bytes_topk, data(s), r, (int)n, n, (int)k, sorted, hist_ready, out.mutable_data_ptr(), k,
+  launch("bytes_topk", bytes_topk, data(s), r, (int)n, n, (int)k, sorted, counted != nullptr, out.mutable_data_ptr(), k,
          w.mutable_data_ptr(), (size_t)w.numel(), st);
   return out;
 }
@@ -381,7 +384,7 @@ Kv kv(const Tensor& q, const Tensor& k, const Tensor& v) {
   return {s, f8};
 }
 
-const Tensor& gather_workspace(const Tensor& q, const QK& s, int64_t kb, bool per_head, long chunk) {
+Tensor gather_workspace(const Tensor& q, const QK& s, int64_t kb, bool per_head, long chunk) {
   need(kb > 0 && kb <= 0x7FFFFFFF);
   size_t n = 0;
   need(bytes_gather_attn_workspace_size(s.B, s.Hq, s.Hk, (int)kb, s.D, per_head, (int)chunk, &n) == 0);
@@ -400,7 +403,7 @@ Tensor gather(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& i
   same_device(q, {&idx});
   const bool per_head = idx.size(1) == s.Hq;
   const int64_t kb = idx.size(2) * page;
-  const Tensor& w = gather_workspace(q, s, kb, per_head, chunk);
+  const Tensor w = gather_workspace(q, s, kb, per_head, chunk);
   Tensor out = empty(q, {s.B, s.Hq, 1, s.D}, at::kBFloat16);
   void* st = stream_of(q);
   launch("bytes_gather_attn", bytes_gather_attn, data(q), data(k), data(v), x.f8, data(idx), out.mutable_data_ptr(),
@@ -426,7 +429,7 @@ Tensor sparse_decode(const Tensor& q, const Tensor& ks, const Tensor* sc, const 
   gather_workspace(q, s, kb, true, 0);
   Tensor scores = empty(q, {s.B, s.Hq, s.S}, at::kFloat);
   score_into(q, ks, sc, zr, bits, scaling, false, scores, nullptr);
-  return gather(q, k, v, topk_of(scores, kb, false, false), scaling, 0, 1, -1);
+  return gather(q, k, v, topk_of(scores, kb, false, nullptr), scaling, 0, 1, -1);
 }
 
 PyObject* token_topk(const Tensor& q, const Tensor& k, const Tensor& v, long kb, double scaling, const Tensor& ks,
@@ -437,11 +440,11 @@ PyObject* token_topk(const Tensor& q, const Tensor& k, const Tensor& v, long kb,
   need(ks.dim() == 4 && ks.size(2) == s.S && ks.size(1) == s.Hk && (sc || ks.sizes() == k.sizes()));
   need((ks.scalar_type() == at::kByte) == (sc != nullptr) && kb >= 1 && kb <= s.S);
   const bool hist = s.B * s.Hk <= 1024;          // rows of the workspace's histogram region
-  const Tensor& w = topk_workspace(q, s.B * s.Hk, s.S, kb);
+  const Tensor w = topk_workspace(q, s.B * s.Hk, s.S, kb);
   gather_workspace(q, s, kb, false, 0);
   Tensor scores = empty(q, {s.B, s.Hk, s.S}, at::kFloat);
   score_into(q, ks, sc, zr, bits, scaling, true, scores, hist ? w.mutable_data_ptr() : nullptr);
-  Tensor idx = topk_of(scores, kb, false, hist);
+  Tensor idx = topk_of(scores, kb, false, hist ? &w : nullptr);
   Tensor out = gather(q, k, v, idx, scaling, 0, 1, -1);
   return Py_BuildValue("(NN)", THPVariable_Wrap(out), THPVariable_Wrap(idx));
 }
@@ -457,7 +460,7 @@ Tensor quest(const Tensor& q, const Tensor& k, const Tensor& v, long kb, double 
   need(pos >= 0 && pos + 1 <= s.S && kb > 0);
   same_device(q, {&kmin, &kmax});
   const int64_t pages = (kb + page - 1) / page, npick = pages < np ? pages : np;
-  const Tensor& w = gather_workspace(q, s, npick * page, true, 0);
+  const Tensor w = gather_workspace(q, s, npick * page, true, 0);
   Tensor bound = empty(q, {s.B, s.Hq, np}, at::kFloat);
   Tensor out = empty(q, {s.B, s.Hq, 1, s.D}, at::kBFloat16);
   void* st = stream_of(q);
@@ -521,7 +524,7 @@ BIND(pq_paged, 9, WRAP(pq_asym(tensor(a[0]), tensor(a[1]), tensor(a[2]), tensor(
 BIND(pq_encode, 2, WRAP(pq_encode(tensor(a[0]), tensor(a[1]))))
 BIND(score_into, 4, (score_into(tensor(a[0]), tensor(a[1]), nullptr, nullptr, 0, number(a[2]), false, tensor(a[3]), nullptr),
                      Py_NewRef(a[3])))
-BIND(topk, 3, WRAP(topk_of(tensor(a[0]), integer(a[1]), a[2] == Py_True, false)))
+BIND(topk, 3, WRAP(topk_of(tensor(a[0]), integer(a[1]), a[2] == Py_True, nullptr)))
 BIND(gather, 8, WRAP(gather(tensor(a[0]), tensor(a[1]), tensor(a[2]), tensor(a[3]), number(a[4]), integer(a[5]),
                             integer(a[6]), a[7] == Py_None ? -1 : row_limit(a[7]))))
 BIND(sparse_decode, 9, WRAP(sparse_decode(tensor(a[0]), tensor(a[1]), optional(a[2]), optional(a[3]), tensor(a[4]),

@@ -243,3 +243,28 @@ def test_dispatch_mode_without_storage_is_refused(dev):
         with pytest.raises(RuntimeError):
             AK.decode_attn_bf16(q, k, v)
     assert torch.equal(AK.decode_attn_bf16(q, k, v), want[0]) and torch.equal(SP.topk_indices(s, 5), want[1])
+
+
+def test_token_topk_counts_and_selects_in_one_buffer(dev):
+    """The selection reads the histogram from the buffer that the score kernel
+    counted into, also where another thread replaces the table's buffer in
+    between: the table is asked for it once."""
+    q, k, v = _qkv(dev, 1, 8, 2, 40000, 64)
+    want = SP.token_topk_decode(q, k, v, 50, 0.1)
+    asked = []
+
+    class Key(tuple):
+        __hash__ = tuple.__hash__
+
+        def __eq__(self, other):
+            asked.append(self[1])
+            return tuple.__eq__(self, other)
+
+    native = _lib.native()
+    native.set_workspaces({Key(n): b for n, b in _lib._ws.items()})
+    try:
+        got = native.token_topk(q, k, v, 50, 0.1, k, None, None, None)
+    finally:
+        native.set_workspaces(_lib._ws)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    assert asked.count("topk") == 1
