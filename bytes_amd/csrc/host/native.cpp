@@ -314,38 +314,52 @@ Tensor pq_encode(const Tensor& x, const Tensor& cb) {
   return idx;
 }
 
-// Scores of keys k (bf16, fp8, or packed codes with scale / zero) into out
-// [B, H, S]; hist: a top-k workspace whose histogram region also counts them.
-void score_into(const Tensor& q, const Tensor& k, const Tensor* sc, const Tensor* zr, long bits, double scaling,
-                bool group_sum, const Tensor& out, void* hist) {
-  const bool packed = sc != nullptr;
+// A score launch whose arguments have been checked.
+struct Score {
   QK s;
   int mode;
   int64_t m0 = 0, m1 = 0, m2 = 0;
-  if (packed) {
+};
+
+// Keys k (bf16, fp8, or packed codes with scale / zero) for the score kernel.
+Score score_of(const Tensor& q, const Tensor& k, const Tensor* sc, const Tensor* zr, long bits, bool group_sum) {
+  Score r;
+  if (sc) {
     need(zr && (bits == 4 || bits == 2) && k.dim() == 4 && k.scalar_type() == at::kByte && k.size(3) * 8 % bits == 0);
-    s = qk(q, k, k.size(3) * 8 / bits);
+    r.s = qk(q, k, k.size(3) * 8 / bits);
     for (const Tensor* t : {sc, zr}) {
-      need(t->scalar_type() == at::kBFloat16 && shape(*t, {s.B, s.Hk, s.S, s.D / 32}));
-      rows(*t, (int)(s.D / 32 * 2));
+      need(t->scalar_type() == at::kBFloat16 && shape(*t, {r.s.B, r.s.Hk, r.s.S, r.s.D / 32}));
+      rows(*t, (int)(r.s.D / 32 * 2));
     }
     need(sc->strides() == zr->strides());
     same_device(q, {sc, zr});
-    mode = bits == 4 ? 2 : 3;
-    m0 = sc->stride(0), m1 = sc->stride(1), m2 = sc->stride(2);
+    r.mode = bits == 4 ? 2 : 3;
+    r.m0 = sc->stride(0), r.m1 = sc->stride(1), r.m2 = sc->stride(2);
   } else {
     need(k.scalar_type() == at::kBFloat16 || k.scalar_type() == kF8);
-    s = qk(q, k);
-    mode = k.scalar_type() == kF8;
+    r.s = qk(q, k);
+    r.mode = k.scalar_type() == kF8;
   }
   rows(k);
-  need(!group_sum || s.Hq / s.Hk <= 16);
+  need(!group_sum || r.s.Hq / r.s.Hk <= 16);
+  return r;
+}
+
+// Scores into out [B, H, S]; hist: a top-k workspace whose histogram region
+// also counts them.
+void score_into(const Score& r, const Tensor& q, const Tensor& k, const Tensor* sc, const Tensor* zr, double scaling,
+                bool group_sum, const Tensor& out, void* hist) {
+  const QK& s = r.s;
   need(out.scalar_type() == at::kFloat && shape(out, {s.B, group_sum ? s.Hk : s.Hq, s.S}) && out.stride(2) == 1);
   void* st = stream_of(q);
-  launch("bytes_sparse_score", bytes_sparse_score, data(q), data(k), mode, packed ? data(*sc) : nullptr,
-         packed ? data(*zr) : nullptr, out.mutable_data_ptr(), s.B, s.Hq, s.Hk, s.S, s.D, group_sum, q.stride(0),
-         q.stride(1), k.stride(0), k.stride(1), k.stride(2), m0, m1, m2, out.stride(0), out.stride(1), (float)scaling,
-         hist, st);
+  launch("bytes_sparse_score", bytes_sparse_score, data(q), data(k), r.mode, sc ? data(*sc) : nullptr,
+         sc ? data(*zr) : nullptr, out.mutable_data_ptr(), s.B, s.Hq, s.Hk, s.S, s.D, group_sum, q.stride(0),
+         q.stride(1), k.stride(0), k.stride(1), k.stride(2), r.m0, r.m1, r.m2, out.stride(0), out.stride(1),
+         (float)scaling, hist, st);
+}
+
+void score_rows(const Tensor& q, const Tensor& k, double scaling, const Tensor& out) {
+  score_into(score_of(q, k, nullptr, nullptr, 0, false), q, k, nullptr, nullptr, scaling, false, out, nullptr);
 }
 
 Tensor topk_workspace(const Tensor& t, int64_t rows_, int64_t n, int64_t k) {
@@ -413,7 +427,8 @@ Tensor gather(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& i
   return out;
 }
 
-// What every launch of a composite needs is looked at before its first one.
+// What every launch of a composite needs is looked at before its first one and
+// before anything is allocated.
 Tensor sparse_decode(const Tensor& q, const Tensor& ks, const Tensor* sc, const Tensor* zr, const Tensor& k,
                      const Tensor& v, double frac, double scaling, long bits) {
   need(bits == 16 ? ks.scalar_type() == at::kBFloat16
@@ -425,10 +440,11 @@ Tensor sparse_decode(const Tensor& q, const Tensor& ks, const Tensor* sc, const 
   const double want = std::nearbyint(frac * (double)s.S);  // round half to even, as Python's round
   need(want <= (double)s.S);
   const int64_t kb = want < 1 ? 1 : (int64_t)want;
+  const Score sco = score_of(q, ks, sc, zr, bits, false);
   topk_workspace(q, s.B * s.Hq, s.S, kb);
   gather_workspace(q, s, kb, true, 0);
   Tensor scores = empty(q, {s.B, s.Hq, s.S}, at::kFloat);
-  score_into(q, ks, sc, zr, bits, scaling, false, scores, nullptr);
+  score_into(sco, q, ks, sc, zr, scaling, false, scores, nullptr);
   return gather(q, k, v, topk_of(scores, kb, false, nullptr), scaling, 0, 1, -1);
 }
 
@@ -439,11 +455,12 @@ PyObject* token_topk(const Tensor& q, const Tensor& k, const Tensor& v, long kb,
   need(s.Hq > s.Hk);                             // idx [B, Hk, kb] is then one list per KV head
   need(ks.dim() == 4 && ks.size(2) == s.S && ks.size(1) == s.Hk && (sc || ks.sizes() == k.sizes()));
   need((ks.scalar_type() == at::kByte) == (sc != nullptr) && kb >= 1 && kb <= s.S);
+  const Score sco = score_of(q, ks, sc, zr, bits, true);
   const bool hist = s.B * s.Hk <= 1024;          // rows of the workspace's histogram region
   const Tensor w = topk_workspace(q, s.B * s.Hk, s.S, kb);
   gather_workspace(q, s, kb, false, 0);
   Tensor scores = empty(q, {s.B, s.Hk, s.S}, at::kFloat);
-  score_into(q, ks, sc, zr, bits, scaling, true, scores, hist ? w.mutable_data_ptr() : nullptr);
+  score_into(sco, q, ks, sc, zr, scaling, true, scores, hist ? w.mutable_data_ptr() : nullptr);
   Tensor idx = topk_of(scores, kb, false, hist ? &w : nullptr);
   Tensor out = gather(q, k, v, idx, scaling, 0, 1, -1);
   return Py_BuildValue("(NN)", THPVariable_Wrap(out), THPVariable_Wrap(idx));
@@ -522,8 +539,7 @@ BIND(pq_asym, 6, WRAP(pq_asym(tensor(a[0]), tensor(a[1]), tensor(a[2]), tensor(a
 BIND(pq_paged, 9, WRAP(pq_asym(tensor(a[0]), tensor(a[1]), tensor(a[2]), tensor(a[3]), tensor(a[4]), &tensor(a[5]),
                                &tensor(a[6]), integer(a[7]), integer(a[8]))))
 BIND(pq_encode, 2, WRAP(pq_encode(tensor(a[0]), tensor(a[1]))))
-BIND(score_into, 4, (score_into(tensor(a[0]), tensor(a[1]), nullptr, nullptr, 0, number(a[2]), false, tensor(a[3]), nullptr),
-                     Py_NewRef(a[3])))
+BIND(score_into, 4, (score_rows(tensor(a[0]), tensor(a[1]), number(a[2]), tensor(a[3])), Py_NewRef(a[3])))
 BIND(topk, 3, WRAP(topk_of(tensor(a[0]), integer(a[1]), a[2] == Py_True, nullptr)))
 BIND(gather, 8, WRAP(gather(tensor(a[0]), tensor(a[1]), tensor(a[2]), tensor(a[3]), number(a[4]), integer(a[5]),
                             integer(a[6]), a[7] == Py_None ? -1 : row_limit(a[7]))))

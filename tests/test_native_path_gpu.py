@@ -268,3 +268,30 @@ def test_token_topk_counts_and_selects_in_one_buffer(dev):
         native.set_workspaces(_lib._ws)
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
     assert asked.count("topk") == 1
+
+
+@pytest.mark.parametrize("shift", ["keys", "scale"])
+def test_composites_refuse_before_they_allocate(dev, shift):
+    """Score keys whose layout needs a copy are left to the wrapper before the
+    score tensor is made."""
+    q, k, v = _qkv(dev, 2, 8, 2, 1000, 64)
+    p, sc, zr = SP.quantize_and_pack_score_keys(k, 4, 32)
+    want = SP.sparse_decode_scalar(q, p, sc, zr, k, v, 0.1, 0.1, score_bits=4)
+    want_t = SP.token_topk_decode(q, k, v, 33, 0.1, k_score=p, score_scale=sc, score_zero=zr, score_bits=4)
+    if shift == "keys":                        # rows off their 16-byte boundary
+        wide = torch.zeros(*p.shape[:3], p.shape[3] + 1, dtype=p.dtype, device=dev)
+        wide[..., 1:] = p
+        p = wide[..., 1:]
+    else:                                      # scale and minimum with strides of their own
+        wide = torch.zeros(*sc.shape[:2], 2 * sc.shape[2], sc.shape[3], dtype=sc.dtype, device=dev)
+        wide[:, :, ::2] = sc
+        sc = wide[:, :, ::2]
+    native = _lib.native()
+    made = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]        # noqa: E731
+    at = made()
+    assert native.sparse_decode(q, p, sc, zr, k, v, 0.1, 0.1, 4) is None
+    assert native.token_topk(q, k, v, 33, 0.1, p, sc, zr, 4) is None
+    assert made() == at
+    assert torch.equal(SP.sparse_decode_scalar(q, p, sc, zr, k, v, 0.1, 0.1, score_bits=4), want)
+    got = SP.token_topk_decode(q, k, v, 33, 0.1, k_score=p, score_scale=sc, score_zero=zr, score_bits=4)
+    assert torch.equal(got[0], want_t[0]) and torch.equal(got[1], want_t[1])
