@@ -42,27 +42,36 @@ def _compile(src: str) -> str:
     return obj
 
 
-def build_native() -> str:
-    """The extension module csrc/host/native.cpp: host code against torch's
-    headers, linked to libbytes_amd.so beside it."""
+def _link(objs: list) -> str:
+    """libbytes_amd.so from the kernels' objects, in the build folder."""
+    out = os.path.join(OBJ, os.path.basename(LIB))
+    r = subprocess.run([HIPCC, "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", out, *objs], capture_output=True,
+                       text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
+    return out
+
+
+def _compile_native() -> str:
+    """The extension module csrc/host/native.cpp, in the build folder: host code
+    against torch's headers, linked to the libbytes_amd.so beside it."""
     import sysconfig
 
     import torch
     from torch.utils import cpp_extension as C
     cxx = os.environ.get("CXX") or shutil.which("g++") or "/opt/rocm/llvm/bin/clang++"
-    tmp = NATIVE + ".tmp"
+    out = os.path.join(OBJ, os.path.basename(NATIVE))
     cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            *(f"-isystem{p}" for p in C.include_paths()), "-isystem/opt/rocm/include",
-           f"-isystem{sysconfig.get_paths()['include']}", os.path.join(CSRC, "host", "native.cpp"), "-o", tmp,
+           f"-isystem{sysconfig.get_paths()['include']}", os.path.join(CSRC, "host", "native.cpp"), "-o", out,
            *(f"-L{p}" for p in C.library_paths()), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip",
-           f"-L{HERE}", "-l:libbytes_amd.so", "-Wl,-rpath,$ORIGIN"]
+           f"-L{OBJ}", f"-l:{os.path.basename(LIB)}", "-Wl,-rpath,$ORIGIN"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"{cxx} failed for csrc/host/native.cpp:\n{r.stdout}\n{r.stderr}")
-    os.replace(tmp, NATIVE)
-    return NATIVE
+    return out
 
 
 def build(verbose: bool = False) -> str:
@@ -73,13 +82,15 @@ def build(verbose: bool = False) -> str:
     workers = max(1, min(len(srcs), int(os.environ.get("MAX_JOBS", os.cpu_count() or 4))))
     with cf.ThreadPoolExecutor(workers) as ex:
         objs = list(ex.map(_compile, srcs))
-    tmp = LIB + ".tmp"
-    cmd = [HIPCC, "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", tmp, *objs]
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    if r.returncode != 0:
-        raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
-    os.replace(tmp, LIB)
-    build_native()
+    lib = _link(objs)
+    native = _compile_native()
+    # both are built: the pair beside this file is replaced as one.  The old
+    # extension goes first, so that none is ever beside a library of another
+    # version, whose entry points may take other arguments.
+    if os.path.exists(NATIVE):
+        os.remove(NATIVE)
+    os.replace(lib, LIB)
+    os.replace(native, NATIVE)
     if verbose:
         print(f"built {LIB} from {len(srcs)} sources and {NATIVE}")
     return LIB
