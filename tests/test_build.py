@@ -1,8 +1,12 @@
-"""The two libraries are published as one (CPU only)."""
+"""The two libraries are published as one, and a native call path that cannot
+be loaded leaves the operators to their Python wrappers (CPU only)."""
+import os
 import subprocess
+import sys
 
 import pytest
 
+from bytes_amd import _lib
 from bytes_amd import build as B
 
 
@@ -40,3 +44,16 @@ def test_build_replaces_both(folder):
     path, _ = folder
     B.build()
     assert (path / "libbytes_amd.so").read_text() == "new" and (path / "_native.so").read_text() == "new"
+
+
+def test_unloadable_native_path_falls_through(monkeypatch):
+    """A missing or mismatched _native.so: one warning that names the build
+    command, and every call goes on in the Python wrapper."""
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.fail(f"{_lib.LIB_PATH} not built (run python -m bytes_amd.build)")
+    monkeypatch.setattr(_lib, "_native", None)
+    monkeypatch.setitem(sys.modules, "bytes_amd._native", None)
+    with pytest.warns(RuntimeWarning, match="python -m bytes_amd.build"):
+        n = _lib.native()
+    assert n.dense(1, 2, 3) is None
+    assert _lib.native() is n
