@@ -39,10 +39,13 @@
 // block-table entries sit in LDS (read from memory, each was a round trip that
 // the V rows behind it waited for), outlier keys stay raw bits until they are
 // used and only 4 of the 16 possible are loaded where 4 suffice, and a row's
-// offset is computed once and passed between lanes.  8 sequences of 2.7K to 8K
-// tokens, H_q 28, H_k 4, D 128, 4 outlier channels, bf16 values, with the merge:
-// 48.2 us without these, 33 with the table, the channels and two tiles, 30 with
-// the offsets and conflict-free LUT stores, 25 with raw outlier keys.
+// offset is computed once and passed between lanes.  The two tiles' registers
+// are used in turn, each refilled once its V rows are staged and the scores
+// taken: with a third set, copied out at a tile's start, the instances of 16
+// outlier channels and bf16 values spilled 40 to 59 VGPRs.  8 sequences of 2.7K
+// to 8K tokens, H_q 28, H_k 4, D 128, bf16 values, with the merge, us for 4 / 8
+// / 16 outlier channels of bf16: 48 / 49 / 59 with one tile in flight and none
+// of these, 25 / 105 / 118 with the third set, 24 / 32 / 44 now.
 //
 // Paged caches (block_table [B, max_blocks] int32, context_lens [B] int32):
 // token t of sequence b is row t % bs of block block_table[b][t / bs]; the
@@ -255,10 +258,10 @@ struct PqCfg {
 //  vc[i]: value code of row p / M, subspace p % M, for staging chunk p = lane + 64*i
 //  vd[i]: dense V chunk p = lane + 64*i (row p / chunks-per-row), bf16 or fp8
 //  ko: the outlier keys of tile row lane % 32, raw bits (OUT of them: 0, 4 or
-//      kPqOutMax; KO4: 4-byte keys).  They are widened where they are used: a
-//      conversion chosen by dtype right after the load would wait for it, and
-//      with it for every V row in flight
-template <int D, bool QV, bool VF8, int OUT, bool KO4>
+//      kPqOutMax; KO: their dtype code).  They are widened where they are used:
+//      a conversion right after the load would wait for it, and with it for
+//      every V row in flight
+template <int D, bool QV, bool VF8, int OUT, int KO>
 struct PqRegs {
   static constexpr int CPR = VF8 ? D / 16 : D / 8;   // 16-byte V chunks per row
   static constexpr int CPL = kTile * CPR / 64;
@@ -270,11 +273,11 @@ struct PqRegs {
 
 // Issue the tile at t0 (rows clamped to len - 1).  Each lane locates its own
 // row lane % 32; rows of the V chunks come from the owning lane by shuffle.
-template <int D, bool QV, bool VF8, int OUT, bool KO4>
+template <int D, bool QV, bool VF8, int OUT, int KO>
 __device__ __forceinline__ void pq_issue(const PqArgs& a, int b, const uint8_t* kih, const uint8_t* vih,
                                          const char* vh, const char* koh, int len, int t0, int lane,
-                                         const PqTable& tab, PqRegs<D, QV, VF8, OUT, KO4>& r) {
-  using R = PqRegs<D, QV, VF8, OUT, KO4>;
+                                         const PqTable& tab, PqRegs<D, QV, VF8, OUT, KO>& r) {
+  using R = PqRegs<D, QV, VF8, OUT, KO>;
   constexpr int M = D / 8;
   int blk, row;
   pq_locate(a, b, min(t0 + (lane & 31), len - 1), blk, row, tab);
@@ -293,7 +296,7 @@ __device__ __forceinline__ void pq_issue(const PqArgs& a, int b, const uint8_t* 
 #pragma unroll
     for (int c = 0; c < OUT; ++c) {
       const int64_t e = o + min(c, a.C - 1);
-      if constexpr (KO4) r.ko[c] = reinterpret_cast<const uint32_t*>(koh)[e];
+      if constexpr (KO == 2) r.ko[c] = reinterpret_cast<const uint32_t*>(koh)[e];
       else r.ko[c] = reinterpret_cast<const uint16_t*>(koh)[e];
     }
   }
@@ -343,9 +346,9 @@ struct CodebookV {
   }
 };
 
-template <int D, bool QV, bool VF8, int OUT, bool KO4>
-__device__ __forceinline__ void pq_stage_dense_v(int lane, const PqRegs<D, QV, VF8, OUT, KO4>& r, char* vst) {
-  using R = PqRegs<D, QV, VF8, OUT, KO4>;
+template <int D, bool QV, bool VF8, int OUT, int KO>
+__device__ __forceinline__ void pq_stage_dense_v(int lane, const PqRegs<D, QV, VF8, OUT, KO>& r, char* vst) {
+  using R = PqRegs<D, QV, VF8, OUT, KO>;
 #pragma unroll
   for (int i = 0; i < R::CPL; ++i) {
     const int p = lane + 64 * i;
@@ -367,11 +370,11 @@ __device__ __forceinline__ void pq_stage_dense_v(int lane, const PqRegs<D, QV, V
 // added, the wave passes the scores through its tile buffer into the
 // score-MFMA layout (head l%16, rows blk*16 + lg*4 + i) and the softmax/PV
 // step runs: quantized V straight from the codebook in LDS, dense V staged in
-// the same buffer first.
-template <int D, bool QV, bool VF8, int OUT, bool KO4>
-__device__ __forceinline__ void pq_tile(const PqArgs& a, const PqRegs<D, QV, VF8, OUT, KO4>& r, uint32_t vmask, int lane,
+// the same buffer first.  refill() is called once r is no longer needed.
+template <int D, bool QV, bool VF8, int OUT, int KO, class REFILL>
+__device__ __forceinline__ void pq_tile(const PqArgs& a, const PqRegs<D, QV, VF8, OUT, KO>& r, uint32_t vmask, int lane,
                                         int nh, const float* lut, const char* vcb, const float* qo, char* vst,
-                                        float& m_run, float& l_run, f32x4 (&acc)[D / 16]) {
+                                        float& m_run, float& l_run, f32x4 (&acc)[D / 16], REFILL refill) {
   constexpr int M = D / 8;
   const int l16 = lane & 15, lg = lane >> 4;
   float* sc_lds = reinterpret_cast<float*>(vst);   // [kPqHeads][32]
@@ -387,13 +390,13 @@ __device__ __forceinline__ void pq_tile(const PqArgs& a, const PqRegs<D, QV, VF8
     const uint32_t code = (w >> ((jj & 3) * 8)) & 0xFFu;
     ps += *reinterpret_cast<const f32x4*>(lut + ((hf * MH + jj) * kPqKMax + code) * kPqHeads);
   }
-  float ko[OUT ? OUT : 1];
+  f32x4 so = {0.f, 0.f, 0.f, 0.f};               // outlier channels, the four heads together
   if constexpr (OUT > 0) {
-    const bool bf = a.ko_dt == 0;
 #pragma unroll
     for (int c = 0; c < OUT; ++c) {
-      if constexpr (KO4) ko[c] = __uint_as_float(r.ko[c]);
-      else ko[c] = bf ? bf16_bits_to_f32((uint16_t)r.ko[c]) : (float)__builtin_bit_cast(_Float16, (uint16_t)r.ko[c]);
+      const float ko = KO == 0 ? bf16_bits_to_f32((uint16_t)r.ko[c])
+                               : KO == 1 ? (float)__builtin_bit_cast(_Float16, (uint16_t)r.ko[c]) : __uint_as_float(r.ko[c]);
+      so += *reinterpret_cast<const f32x4*>(qo + c * kPqHeads) * ko;   // zero past C
     }
   }
   f32x4 sc4;
@@ -401,13 +404,8 @@ __device__ __forceinline__ void pq_tile(const PqArgs& a, const PqRegs<D, QV, VF8
   for (int h = 0; h < kPqHeads; ++h) {
     const float o = shfl_xor_f(ps[h], 32);
     sc4[h] = hf ? o + ps[h] : ps[h] + o;
-    if constexpr (OUT > 0) {
-      float so = 0.f;
-#pragma unroll
-      for (int c = 0; c < OUT; ++c) so += qo[h * kPqOutMax + c] * ko[c];   // zero past C
-      sc4[h] += so;
-    }
   }
+  if constexpr (OUT > 0) sc4 += so;
 #pragma unroll
   for (int rep = 0; rep < 2; ++rep) {
     const int h = hf * 2 + rep;
@@ -427,7 +425,8 @@ __device__ __forceinline__ void pq_tile(const PqArgs& a, const PqRegs<D, QV, VF8
   } else {
     // V tile into the same buffer
     wave_lds_sync();
-    pq_stage_dense_v<D, QV, VF8, OUT, KO4>(lane, r, vst);
+    pq_stage_dense_v<D, QV, VF8, OUT, KO>(lane, r, vst);
+    refill();
     wave_lds_sync();
     tile_softmax_pv<D, false>(s, l16 < nh ? vmask : 0u, a.scale_log2, lane, vst, m_run, l_run, acc);
   }
@@ -448,10 +447,10 @@ __device__ __forceinline__ void stage_chunks(int n, SRC src, DST dst) {
   }
 }
 
-template <int D, bool BUILD_LUT, bool QV, bool VF8, int OUT, bool KO4>
+template <int D, bool BUILD_LUT, bool QV, bool VF8, int OUT, int KO>
 __global__ __launch_bounds__(kPqWaves * 64, 1) void pq_decode_kernel(PqArgs a) {
   using C = PqCfg<D, QV>;
-  using Regs = PqRegs<D, QV, VF8, OUT, KO4>;
+  using Regs = PqRegs<D, QV, VF8, OUT, KO>;
   constexpr int M = D / 8;
   __shared__ __attribute__((aligned(16))) char smem_raw[C::kSmem];
   float* lut = reinterpret_cast<float*>(smem_raw);
@@ -495,7 +494,7 @@ __global__ __launch_bounds__(kPqWaves * 64, 1) void pq_decode_kernel(PqArgs a) {
       tab_lds[e] = min(max(a.btab[(int64_t)b * a.bt_sb + tab_q0 + e], 0), a.nblk - 1);
   }
   Regs r;
-  if (any) pq_issue<D, QV, VF8, OUT, KO4>(a, b, kih, vih, vh, koh, len, t, lane, tab, r);
+  if (any) pq_issue<D, QV, VF8, OUT, KO>(a, b, kih, vih, vh, koh, len, t, lane, tab, r);
 
   // The value codebook (quantized V) is requested now, with the first tile's
   // codes, so it arrives while the LUTs are built or staged; it is stored to
@@ -584,7 +583,7 @@ __global__ __launch_bounds__(kPqWaves * 64, 1) void pq_decode_kernel(PqArgs a) {
   float* qo = reinterpret_cast<float*>(smem_raw + C::LUT + C::VCB + kPqWaves * C::TILE);
   if constexpr (OUT > 0) {
     for (int e = threadIdx.x; e < kPqHeads * kPqOutMax; e += kPqWaves * 64) {
-      const int h = e / kPqOutMax, c = e - h * kPqOutMax;
+      const int c = e / kPqHeads, h = e - c * kPqHeads;     // a channel's heads adjacent, as the LUT's
       qo[e] = (h < nh && c < a.C) ? load_any(a.qout, a.qo_dt, (int64_t)b * a.qo_sb + (int64_t)(hq0 + h) * a.qo_sh + c)
                                   : 0.f;
     }
@@ -597,27 +596,28 @@ __global__ __launch_bounds__(kPqWaves * 64, 1) void pq_decode_kernel(PqArgs a) {
 
   __syncthreads();
   if (any) {
-    // tile t runs on the registers that arrived during the last tiles, which
-    // are copied out first and refilled with a tile further on (clamped past
-    // the end): the next one, or with dense values the one after it, so two
-    // tiles of V rows are in flight per wave
+    // tile t runs on the registers that arrived during the last tiles (rows
+    // past the end clamped): copied out first and refilled with the next tile,
+    // or with dense values two sets in turn, each refilled with the tile after
+    // the next one as soon as it has been read
     if constexpr (QV) {
       for (; t < t_end; t += STEP) {
         const Regs cur = r;
-        pq_issue<D, QV, VF8, OUT, KO4>(a, b, kih, vih, vh, koh, len, t + STEP, lane, tab, r);
+        pq_issue<D, QV, VF8, OUT, KO>(a, b, kih, vih, vh, koh, len, t + STEP, lane, tab, r);
         wave_lds_sync();
-        pq_tile<D, QV, VF8, OUT, KO4>(a, cur, range_mask(t, t_end), lane, nh, lut, vcb, qo, vst, m_run, l_run, acc);
+        pq_tile<D, QV, VF8, OUT, KO>(a, cur, range_mask(t, t_end), lane, nh, lut, vcb, qo, vst, m_run, l_run, acc,
+                                     [] {});
       }
     } else {
       // (rows clamped to t_end - 1, the last token of the staged entries)
       tab = PqTable{tab_lds, tab_q0, tab_n};
       Regs r1;
-      pq_issue<D, QV, VF8, OUT, KO4>(a, b, kih, vih, vh, koh, t_end, t + STEP, lane, tab, r1);
+      pq_issue<D, QV, VF8, OUT, KO>(a, b, kih, vih, vh, koh, t_end, t + STEP, lane, tab, r1);
       auto step = [&](Regs& x) {
-        const Regs cur = x;
-        pq_issue<D, QV, VF8, OUT, KO4>(a, b, kih, vih, vh, koh, t_end, t + 2 * STEP, lane, tab, x);
         wave_lds_sync();
-        pq_tile<D, QV, VF8, OUT, KO4>(a, cur, range_mask(t, t_end), lane, nh, lut, vcb, qo, vst, m_run, l_run, acc);
+        pq_tile<D, QV, VF8, OUT, KO>(a, x, range_mask(t, t_end), lane, nh, lut, vcb, qo, vst, m_run, l_run, acc, [&] {
+          pq_issue<D, QV, VF8, OUT, KO>(a, b, kih, vih, vh, koh, t_end, t + 2 * STEP, lane, tab, x);
+        });
         t += STEP;
         return t < t_end;
       };
@@ -1508,19 +1508,21 @@ static int pq_launch(PqArgs& a, int mode, bool vf8, int B, int Hq, int Hk, int S
   splitk_carve(workspace, units, ns, a.o);
   dim3 grid((unsigned)(ns * units)), block(kPqWaves * 64);
   // outlier channels a tile keeps per row: none, up to 4, up to kPqOutMax
-#define PQ_LAUNCH(DD, BL, QQ, F8, OU, K4) \
-  BYTES_LAUNCH(kProfPq, (pq_decode_kernel<DD, BL, QQ, F8, OU, K4>), grid, block, 0, st, a)
-#define PQ_OUT(DD, F8)                                                      \
-  if (a.C == 0) PQ_LAUNCH(DD, false, false, F8, 0, false);                  \
-  else if (a.C <= 4 && a.ko_dt != 2) PQ_LAUNCH(DD, false, false, F8, 4, false); \
-  else if (a.C <= 4) PQ_LAUNCH(DD, false, false, F8, 4, true);              \
-  else if (a.ko_dt != 2) PQ_LAUNCH(DD, false, false, F8, kPqOutMax, false); \
-  else PQ_LAUNCH(DD, false, false, F8, kPqOutMax, true);
-#define PQ_MODES(DD)                                                  \
-  if (mode == 0) PQ_LAUNCH(DD, false, true, false, 0, false);         \
-  else if (mode == 2) PQ_LAUNCH(DD, true, false, false, 0, false);    \
-  else if (mode == 3) PQ_LAUNCH(DD, true, true, false, 0, false);     \
-  else if (!vf8) { PQ_OUT(DD, false) }                                \
+#define PQ_LAUNCH(DD, BL, QQ, F8, OU, KO) \
+  BYTES_LAUNCH(kProfPq, (pq_decode_kernel<DD, BL, QQ, F8, OU, KO>), grid, block, 0, st, a)
+#define PQ_KO(DD, F8, OU)                                          \
+  if (a.ko_dt == 0) PQ_LAUNCH(DD, false, false, F8, OU, 0);        \
+  else if (a.ko_dt == 1) PQ_LAUNCH(DD, false, false, F8, OU, 1);   \
+  else PQ_LAUNCH(DD, false, false, F8, OU, 2);
+#define PQ_OUT(DD, F8)                                  \
+  if (a.C == 0) PQ_LAUNCH(DD, false, false, F8, 0, 0);  \
+  else if (a.C <= 4) { PQ_KO(DD, F8, 4) }               \
+  else { PQ_KO(DD, F8, kPqOutMax) }
+#define PQ_MODES(DD)                                              \
+  if (mode == 0) PQ_LAUNCH(DD, false, true, false, 0, 0);         \
+  else if (mode == 2) PQ_LAUNCH(DD, true, false, false, 0, 0);    \
+  else if (mode == 3) PQ_LAUNCH(DD, true, true, false, 0, 0);     \
+  else if (!vf8) { PQ_OUT(DD, false) }                            \
   else { PQ_OUT(DD, true) }
   if (D == 128) {
     PQ_MODES(128)
@@ -1529,6 +1531,7 @@ static int pq_launch(PqArgs& a, int mode, bool vf8, int B, int Hq, int Hk, int S
   }
 #undef PQ_MODES
 #undef PQ_OUT
+#undef PQ_KO
 #undef PQ_LAUNCH
   int rc = (int)hipGetLastError();
   if (rc) return rc;
