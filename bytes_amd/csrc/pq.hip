@@ -447,8 +447,12 @@ __device__ __forceinline__ void stage_chunks(int n, SRC src, DST dst) {
   }
 }
 
+// D = 64 leaves LDS for two workgroups per CU (70 KB each): four waves to a
+// SIMD, at most 128 VGPRs, wherever that needs no spills (up to 4 outlier
+// channels).  Without outliers, 134 VGPRs and one workgroup, B32 H_q 64 H_k 8
+// L4096 bf16 took 42 us, 35 with two.
 template <int D, bool BUILD_LUT, bool QV, bool VF8, int OUT, int KO>
-__global__ __launch_bounds__(kPqWaves * 64, 1) void pq_decode_kernel(PqArgs a) {
+__global__ __launch_bounds__(kPqWaves * 64, D == 64 && OUT <= 4 ? 4 : 1) void pq_decode_kernel(PqArgs a) {
   using C = PqCfg<D, QV>;
   using Regs = PqRegs<D, QV, VF8, OUT, KO>;
   constexpr int M = D / 8;

@@ -54,3 +54,16 @@ def _notes(elf):
 def test_no_kernel_spills_vector_registers():
     spilled = {n: k[".vgpr_spill_count"] for n, k in _kernels().items() if k[".vgpr_spill_count"]}
     assert not spilled, spilled
+
+
+def test_narrow_pq_decode_leaves_room_for_two_workgroups():
+    """The D = 64 general PQ kernel (eight waves a workgroup) with at most 4
+    outlier channels: four waves to a SIMD, and twice its LDS, fit a CU."""
+    seen = 0
+    for n, k in _kernels().items():
+        m = re.search(r"pq_decode_kernelILi64ELb\dELb\dELb\dELi([04])E", n)
+        if m:
+            seen += 1
+            regs = -(-(k[".vgpr_count"] + k.get(".agpr_count", 0)) // 8) * 8
+            assert regs <= 128 and 2 * k[".group_segment_fixed_size"] <= 160 * 1024, n
+    assert seen
