@@ -603,8 +603,10 @@ __global__ __launch_bounds__(kPqWaves * 64, D == 64 && OUT <= 4 ? 4 : 1) void pq
     // tile t runs on the registers that arrived during the last tiles (rows
     // past the end clamped): copied out first and refilled with the next tile,
     // or with dense values two sets in turn, each refilled with the tile after
-    // the next one as soon as it has been read
-    if constexpr (QV) {
+    // the next one as soon as it has been read.  (Mode 2, whose LUTs are built
+    // from the codebook, keeps one: at D 128 B1 H_q 28 L32K, four tiles a wave,
+    // 19.9 us with one and 21.1 with two, B32 H_q 64 L4096 67.6 and 66.8.)
+    if constexpr (QV || BUILD_LUT) {
       for (; t < t_end; t += STEP) {
         const Regs cur = r;
         pq_issue<D, QV, VF8, OUT, KO>(a, b, kih, vih, vh, koh, len, t + STEP, lane, tab, r);
