@@ -845,10 +845,20 @@ int bytes_sparse_score(const void* q, const void* k, int k_mode, const void* k_s
       ((int64_t)S + 64) * k_ss * (k_mode == kKeyBf16 ? 2 : 1) >= ((int64_t)1 << 32))
     return (int)hipErrorNotSupported;
   a.scaling = scaling;
-  // many heads per KV head (folded query chunks), output rows on 16-byte
-  // boundaries: the block kernel
-  if (k_mode == kKeyBf16 && !a.group_sum && a.G >= kScoreBlockHeads && reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
-      o_sb % 4 == 0 && o_sh % 4 == 0) {
+  // Many heads per KV head (folded query chunks), output rows on 16-byte
+  // boundaries: the block kernel, about four workgroups per CU (the keys' first
+  // loads of some overlap the stores of others), where that gives a workgroup
+  // two or more blocks of heads for its keys.  With one each it reads the keys
+  // as often as the streaming kernel does, whose loads are better spread: D 128
+  // 224 heads x 4 x 4096 keys (896 blocks of 16 heads x 256 tokens) 12.4 us
+  // streaming, 14.4 here, 64 x 32768 (512) 7.3 and 8.2; from the line on 96 x 4 x
+  // 16384 (1536) 23.5 and 14.3.  D = 64 also gains where the grid is at most one
+  // workgroup per CU, from its fewer instructions (256 x 2048, 128 blocks 4.3
+  // and 3.5; 224 x 2 x 8192, 896 blocks 8.6 and 9.6).
+  const int tparts = (S + kScoreWaves * 64 - 1) / (kScoreWaves * 64);
+  const long blocks = (long)B * Hk * tparts * ((a.G + 15) / 16), cus = device_cu_count(), want = 4 * cus;
+  if (k_mode == kKeyBf16 && !a.group_sum && a.G >= kScoreBlockHeads && (blocks > want || (D == 64 && blocks <= cus)) &&
+      reinterpret_cast<uintptr_t>(out) % 16 == 0 && o_sb % 4 == 0 && o_sh % 4 == 0) {
     ScoreBlockArgs c;
     c.q = a.q; c.q_sb = q_sb; c.q_sh = q_sh;
     c.k = static_cast<const uint16_t*>(k);
@@ -857,10 +867,7 @@ int bytes_sparse_score(const void* q, const void* k, int k_mode, const void* k_s
     c.Hk = Hk; c.G = a.G; c.S = S;
     c.HB = (a.G + 15) / 16;
     c.scaling = scaling;
-    c.tparts = (S + kScoreWaves * 64 - 1) / (kScoreWaves * 64);
-    // about four workgroups per CU, so the keys' first loads of some overlap
-    // the stores of others
-    const long blocks = (long)B * Hk * c.tparts * c.HB, want = 4L * device_cu_count();
+    c.tparts = tparts;
     const long hpw = (blocks + want - 1) / want;
     c.hpw = (int)(hpw < c.HB ? hpw : c.HB);
     c.hgroups = (c.HB + c.hpw - 1) / c.hpw;

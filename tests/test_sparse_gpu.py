@@ -409,3 +409,22 @@ def test_score_many_heads_per_kv_head(dev, B, Hk, G, S, D):
     lo = 4 if wide.shape[2] >= S + 4 else 0
     assert torch.equal(wide[:, :, lo:lo + S], got)
     assert (wide[:, :, :lo] == 7).all() and (wide[:, :, lo + S:] == 7).all()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,Hk,G,S", [(2, 2, 70, 13200),       # 1040 blocks of 16 heads x 256 tokens: two a workgroup
+                                      (1, 1, 520, 8200),       # 1089, a head block of 8
+                                      (1, 2, 64, 8192),        # 256: at most one workgroup per CU
+                                      (1, 1, 64, 65536)])      # 1024: one block a workgroup
+def test_score_many_heads_rule(dev, B, Hk, G, S, D):
+    """Both sides of the lines between the block and the streaming kernel: the
+    same bits as 16 heads at a time."""
+    g = torch.Generator(device=dev).manual_seed(S + G)
+    q = torch.randn(B, Hk * G, 1, D, generator=g, device=dev).to(torch.bfloat16)
+    k = torch.randn(B, Hk, S, D, generator=g, device=dev).to(torch.bfloat16)
+    got = SP.sparse_score_scalar(q, k, 0.3).reshape(B, Hk, G, S)
+    qg = q.reshape(B, Hk, G, 1, D)
+    for h0 in range(0, G, 16):
+        n = min(16, G - h0)
+        part = SP.sparse_score_scalar(qg[:, :, h0:h0 + n].reshape(B, Hk * n, 1, D), k, 0.3)
+        assert torch.equal(got[:, :, h0:h0 + n], part.reshape(B, Hk, n, S)), h0
