@@ -15,12 +15,17 @@
 // (the first wave's first keys, searched in that wave alone), the second lies
 // past the k-th key by the sample's spacing, and from then on the trial
 // interpolates between the bracket's counts in key space; where that shrank
-// the bracket by less than half it takes the middle key, and so does every
-// trial from the twelfth count on, so at most 44 counts are ever needed
-// (five or six on ordinary scores, about 30 where most scores are equal to
-// others).  The selection's membership masks are then taken by wave ballots,
-// and each thread lists its PER consecutive elements from them, so the output
-// is in index order whatever the striping.
+// the bracket by less than half it takes the middle key.  Five or six counts
+// find the key of ordinary scores.  After kRowCounts of them (scores that are
+// mostly equal to others, or far from a line in key space) the bracket's ends
+// are moved to its own smallest and largest key, and again whenever a trial
+// falls between two values, so each value is told apart by one count; every
+// trial from the twenty-first on takes the middle key, so at most 53 counts are
+// ever needed.  2048 rows of 16384, k = 1638, us: normal scores 46, integers
+// from -8 to 8 51, rounded to bf16 49 (with trials alone, some 30 counts, 99 and
+// 85).  The selection's membership masks are then taken by wave ballots, and
+// each thread lists its PER consecutive elements from them, so the output is in
+// index order whatever the striping.
 #pragma once
 #include "wave_select.h"
 
@@ -84,6 +89,37 @@ struct RowBracket {
   uint32_t lo, hi, cl, ch;             // cl = count(>= lo) >= k > ch = count(> hi)
   bool slow;                           // the last interpolation shrank the bracket by less than half
 };
+
+constexpr int kRowCounts = 7;          // interpolated counts before the bracket is snapped to its keys
+
+// Moves the bracket's ends to the smallest and the largest key between them.
+template <int NT, int PER, class L>
+__device__ __forceinline__ void row_snap(const uint32_t (&key)[PER], RowBracket& b, L& lds, int& turn) {
+  uint32_t up = 0xFFFFFFFFu, down = 0xFFFFFFFFu; // distances; keys outside wrap past those inside
+#pragma unroll
+  for (int q = 0; q < PER; ++q) {
+    up = min(up, key[q] - b.lo);
+    down = min(down, b.hi - key[q]);
+  }
+  down = ~down;                                  // complemented: one minimum and one maximum
+  wave_minmax_u32(up, down);
+  if constexpr (NT > 64) {
+    constexpr int NW = NT / 64;
+    turn ^= 1;
+    if ((threadIdx.x & 63) == 0) {
+      lds.red[turn][threadIdx.x >> 6] = up;
+      lds.red[turn][NW + (threadIdx.x >> 6)] = down;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      up = min(up, lds.red[turn][w]);
+      down = max(down, lds.red[turn][NW + w]);
+    }
+  }
+  b.lo += (uint32_t)__builtin_amdgcn_readfirstlane((int)up);
+  b.hi -= (uint32_t)__builtin_amdgcn_readfirstlane((int)~down);
+}
 
 // A trial key in (lo, hi] (lo < hi): where a line through the bracket's counts
 // reaches k, in key space (which is linear in the score within a binade); the
@@ -172,8 +208,11 @@ __device__ __forceinline__ RowSel row_search(const uint32_t (&key)[PER], int n, 
   RowBracket b{1u, 0xFFFFFFFFu, (uint32_t)n, 0u, false};
   if ((uint32_t)n > k) {
     gap *= 1.5f;
-    for (int i = 0;; ++i) {
-      if (row_update(b, t, row_sum<NT>(wave_count_ge<PER>(key, t), lds, turn), k)) break;
+    int i = 0;
+    bool done = false;
+    for (; i < kRowCounts; ++i) {
+      done = row_update(b, t, row_sum<NT>(wave_count_ge<PER>(key, t), lds, turn), k);
+      if (done) break;
       if (i < 4 && (b.lo == 1u || b.hi == 0xFFFFFFFFu)) {
         // one side only so far: past the k-th key by the sample's spacing
         const bool up = b.hi == 0xFFFFFFFFu;
@@ -183,7 +222,18 @@ __device__ __forceinline__ RowSel row_search(const uint32_t (&key)[PER], int n, 
         gap *= 4.f;
         b.slow = false;
       } else {
-        t = row_trial(b, k, i >= 11);
+        t = row_trial(b, k, false);
+      }
+    }
+    if (__builtin_expect(!done, 0)) {
+      for (uint32_t in = 0u;; ++i) {
+        if (in == 0u || b.cl - b.ch == in) {
+          row_snap<NT, PER>(key, b, lds, turn);
+          if (b.lo >= b.hi) break;
+        }
+        in = b.cl - b.ch;
+        t = row_trial(b, k, i >= 20);
+        if (row_update(b, t, row_sum<NT>(wave_count_ge<PER>(key, t), lds, turn), k)) break;
       }
     }
   }

@@ -428,3 +428,28 @@ def test_score_many_heads_rule(dev, B, Hk, G, S, D):
         n = min(16, G - h0)
         part = SP.sparse_score_scalar(qg[:, :, h0:h0 + n].reshape(B, Hk * n, 1, D), k, 0.3)
         assert torch.equal(got[:, :, h0:h0 + n], part.reshape(B, Hk, n, S)), h0
+
+
+@pytest.mark.parametrize("rows,n", [(300, 4097), (300, 8192), (4, 8193), (32, 9000), (33, 9000), (40, 12287),
+                                    (40, 12288), (3, 16384), (300, 16384), (260, 32768), (256, 65536)])
+def test_topk_rows_past_the_first_counts(dev, rows, n):
+    """Rows whose k-th score the interpolated counts do not find: few distinct
+    values, neighbouring ones, values far from a line in key space and ordered
+    rows, on both sides of the row and length rules, against a stable sort."""
+    g = torch.Generator(device=dev).manual_seed(n + rows)
+    x = torch.randn(rows, n, generator=g, device=dev)
+    at = torch.arange(n, device=dev)
+    ulp = torch.randint(0, 3, (rows, n), generator=g, device=dev)
+    kinds = {"integers": (2 * x).round(),
+             "bf16": x.to(torch.bfloat16).float(),
+             "neighbours": (1.0 + ulp * 2.0 ** -23),
+             "two values": torch.where(x > 1, 3e30, -1e-30),
+             "wide": torch.exp(40 * x).clamp(1e-37, 1e37) * torch.sign(x),
+             "ascending": x.sort(1).values,
+             "masked": x.masked_fill(at >= n // 20, -math.inf),
+             "far from the sample": torch.where(at < n // 2, x, x * 1e-6 + 50)}
+    for kind, s in kinds.items():
+        want = torch.sort(s, dim=1, descending=True, stable=True).indices
+        for k in (1, 65, n // 10, n - 1):
+            got = SP.topk_indices(s, k, sorted=False).long()
+            assert torch.equal(got, want[:, :k].sort(1).values), (kind, k)
