@@ -1080,10 +1080,17 @@ static int topk_launch(const float* scores, int64_t rows, int n, int64_t row_str
   // elements: 64 rows of 5000 11.7 us there against 13.9, 2048 rows of 8192
   // 91 against 29) or spread over several workgroups a row (above 16384: 128
   // rows of 65536 32.5 against 37.6, 256 rows 49.5 against 41.9; sorted, 300
-  // rows 65 against 72).  Rows of 8193 to 16384 gain at any count (4 rows of
-  // 16384: 19.3 against 13.6).
+  // rows 65 against 72).  Rows of 8193 to 16384 gain at any count from 12288 on
+  // (64 rows 14.9 against 13.2, of 16384 17.9 against 13.5; means over normal,
+  // exponential and bf16-rounded scores, k = n / 10 and 64) and below that up to
+  // 32 rows (4 rows of 9000 13.2 against 11.0, 32 rows 13.3 against 13.1); with
+  // more, up to the CUs, the row that needs the most counts takes longer than
+  // the digit passes (128 rows of 9000 13.5 against 14.0, single sets to 16.4).
   const int cus = device_cu_count();
-  const bool row_regs = n <= 8192 ? rows > cus : n <= kShortRow ? true : n <= kRowMax && rows >= (sorted ? 2 : 1) * cus;
+  const bool row_regs = n <= 8192    ? rows > cus
+                        : n < 12288  ? rows > cus || rows <= 32
+                        : n <= kShortRow ? true
+                                         : n <= kRowMax && rows >= (sorted ? 2 : 1) * cus;
   if (row_regs && (!sorted || k <= kRowSortK)) {
     if (rows > 0x7FFFFFFFL) return (int)hipErrorInvalidConfiguration;
     uint32_t* gh = hist_ready ? ws.hist : nullptr;
