@@ -235,3 +235,45 @@ def test_attend_topk_list_dtypes(dev, fp8):
         assert torch.equal(got, SA.attend_topk(qd, kd, vd, wide[..., :ksel], pos, 0.125))
         if not fp8:
             _check(got, R.attend_topk(q, k, v, idx.clamp(-3, S + 9), pos, 0.125), f"attend S {S}")
+
+
+@pytest.mark.parametrize("last", [False, True])
+@pytest.mark.parametrize("nrun", [0, 300])
+def test_select_step_nonfinite(dev, last, nrun):
+    """One fused step on scores of NaN (both signs), infinities, zeros of both
+    signs and ties, inside and past the causal limit and inside the recent
+    window, against the mask, top-k and merge launches."""
+    from bytes_amd._lib import call, ptr, stream_of
+    Qc, rows, n, kb, S, kc0, local_w = 6, 12, 1001, 300, 4000, 1500, 40
+    W, kbp = 1408, 320
+    g = torch.Generator().manual_seed(7)
+    x = torch.randn(rows, W, generator=g)
+    special = torch.tensor([float("nan"), 0.0, float("inf"), -float("inf"), 0.0, -0.0, 1.0])
+    special[1] = torch.tensor([-0x400000], dtype=torch.int32).view(torch.float32)[0]      # a negative NaN
+    pick = torch.randint(0, 60, (rows, W), generator=g)
+    x = torch.where(pick < 7, special[pick.clamp_max(6)], x)
+    x[rows - 1] = float("nan")
+    x[rows - 2] = -float("inf")
+    x = x.to(dev)
+    pos = torch.tensor([3, kc0 - 1, kc0, kc0 + 20, kc0 + n // 2, S - 1], device=dev)
+    ridx = torch.stack([torch.randperm(kc0, generator=g)[:kb].sort().values for _ in range(rows)]).int().to(dev)
+    ridx[0, 100:] = S                          # fillers
+    off, st = kbp - nrun, stream_of(x)
+    ksel = min(kb, nrun + n)
+    # the separate launches
+    y = x.clone()
+    call("bytes_select_mask_at", ptr(y) + 4 * kbp, rows, n, W, kc0, ptr(pos), Qc, 1, local_w, st)
+    sel = SP.topk_indices(y[:, off:off + nrun + n].contiguous(), ksel, sorted=last)
+    v1, i1 = torch.zeros_like(x), torch.zeros(rows, kb, dtype=torch.int32, device=dev)
+    call("bytes_select_merge", ptr(y), W, off, nrun, ptr(ridx), kb, ptr(sel), sel.stride(0), ksel, kc0, S, rows,
+         None if last else ptr(v1), W, kbp - kb, ptr(i1), kb, kb, st)
+    # the fused one
+    v2, i2 = torch.zeros_like(x), torch.zeros(rows, kb, dtype=torch.int32, device=dev)
+    out = torch.zeros(rows, kb, dtype=torch.int64, device=dev) if last else None
+    call("bytes_select_step", ptr(x), W, off, nrun, n, ptr(ridx), kb, kc0, ptr(pos), Qc, local_w, S, kb, rows,
+         ptr(v2), W, kbp - kb, ptr(i2), kb, ptr(out) if last else None, st)
+    if last:
+        assert torch.equal(out, SA._fill(i1, pos, Qc, S, kb, torch.int64))
+    else:
+        assert torch.equal(i2, i1)
+        assert torch.equal(v2.view(torch.int32), v1.view(torch.int32))
