@@ -4,16 +4,18 @@
 // arguments that need no conversion or copy: check them, allocate the output,
 // find the workspace and call the C ABI on the current stream.  Anything else
 // (a wrong shape or dtype, rows off their 16-byte boundary, a tensor subclass
-// or a functorch wrapper, a workspace that is missing or too small, a size the
-// library refuses) returns None before anything is allocated or launched, and
-// the wrapper goes on in Python, where the copies, the workspace and the error
-// messages are.  No state is kept here: workspaces are looked up in the
+// or a functorch wrapper, a workspace that is missing or too small, a size its
+// query refuses) returns None before anything is allocated or launched, and the
+// wrapper goes on in Python, where the copies, the workspace and the error
+// messages are.  (So does an output that a dispatch mode gave no memory, before
+// anything is launched.)  No state is kept here: workspaces are looked up in the
 // package's own table on every call.  The GIL is released while the library
 // launches, as ctypes does.
 //
 // Why: a decode step of a few microseconds was bound by its wrapper's Python
-// (host time per call, us: dense decode 21, KIVI 33, PQ 28, Quest 41, of which
-// the launches themselves take 4 to 6).
+// (eager calls in a row, us a call: dense decode B1 8K 21, KIVI B4 16K 29, PQ
+// B1 32K 26, Quest B1 32K 38, of which the launches themselves take 4 to 6; 8,
+// 13, 10 and 18 from here).
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 

@@ -1401,7 +1401,9 @@ struct PipeMeta {
 // all start early and end together.  With each unit's residual splits after its
 // quantized ones, the quantized splits that these displaced from the first pass
 // started only when others had ended: 4-bit B32 H_k8 L16K, 512 quantized splits
-// on 512 slots, 176 us then and 137 now (129 with no residual window).
+// on 512 slots, a step of 199 us then and 161 now, B1 H_k4 L128K 29.5 and 25.4
+// (2-bit 24.8 and 21.9).  Where the residual splits are few the order matters
+// little: 4-bit B4 H_k4 L64K 38.1 and 37.9, L32K 23.6 and 24.1.
 __device__ __forceinline__ UnitLoc pipe_locate(const KiviArgs& a) {
   const int L = blockIdx.x, nr = a.o.nwg - a.nquant;
   if (L < nr) {

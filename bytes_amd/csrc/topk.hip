@@ -707,8 +707,8 @@ __global__ __launch_bounds__(kSmallThreads) void topk_small_kernel(const float* 
 // us per call at 2048 rows, unsorted, here against the paths of the same
 // shapes without it (one 1024-thread workgroup re-reading the row for three
 // digit passes and the collection up to 16384, else histogram, filter and
-// select launches): n = 8192 k = 410 29 / 91, 16384 k = 819 48 / 154, 32768
-// k = 1638 88 / 196, 65536 k = 655 192 / 287.
+// select launches): n = 8192 k = 410 27 / 89, 16384 k = 819 44 / 144, 32768
+// k = 1638 83 / 185, 65536 k = 655 197 / 288.
 constexpr int kRowSortK = 1024;
 constexpr int kRowMax = 65536;         // 1024 threads x 64 keys
 
@@ -1078,7 +1078,7 @@ static int topk_launch(const float* scores, int64_t rows, int n, int64_t row_str
   // longer rows that one workgroup's registers hold, where the rows alone keep
   // the chip busy; fewer rows finish sooner on 16 waves a row (up to 8192
   // elements: 64 rows of 5000 11.7 us there against 13.9, 2048 rows of 8192
-  // 91 against 29) or spread over several workgroups a row (above 16384: 128
+  // 89 against 27) or spread over several workgroups a row (above 16384: 128
   // rows of 65536 32.5 against 37.6, 256 rows 49.5 against 41.9; sorted, 300
   // rows 65 against 72).  Rows of 8193 to 16384 gain at any count from 12288 on
   // (64 rows 14.9 against 13.2, of 16384 17.9 against 13.5; means over normal,
